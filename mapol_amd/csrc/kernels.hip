@@ -523,7 +523,7 @@ struct FactorPlan {
   // lane) and for the form that reads operands from memory (up to 4)
   int tjobs_s, tjobs_g;
   const int2 *tjob_s, *tjob_g;
-  int tail_mfma;                       // FP32 tail inverse on matrix cores
+  int tail_mfma;                       // tail inverse on matrix cores (1024 lanes)
   // the forward substitution's outputs run while at most this many
   // instances of the batch are active (-1: never); the solve then starts
   // from them (same limit in the solve plan)
@@ -772,160 +772,271 @@ __device__ __forceinline__ bool pair_inv(const B4<T> (&m)[2][2], B4<T> (&r)[2][2
   return bad;
 }
 
-// Dense-tail inverse on matrix cores (FP32, workgroups of 1024 lanes).  S,
-// 2s scalars per side, is taken as one 128 x 128 matrix (identity beyond
-// S, zero coupling); wave w holds the 32 x 32 tile (w / 4, w % 4) in the
-// accumulators of v_mfma_f32_32x32x2f32 for the whole elimination
-// (accumulator v of lane l: tile row 8 (v / 4) + 4 (l / 32) + v % 4, tile
-// column l % 32; operand lane l: A row / B column l % 32, k = l / 32).
-// Gauss-Jordan by pivot quads, the block pivots 2p and 2p + 1 (scalars
-// 4p..4p+3), in the order of the block form.  A step updates every entry by
-// one rank-4 product,
+// Dense-tail inverse on matrix cores (workgroups of 1024 lanes).  S, 2s scalars
+// per side, is taken as one 128 x 128 matrix (identity beyond S, zero
+// coupling); wave w holds the 32 x 32 tile (w / 4, w % 4) as 2 x 2 accumulators
+// of a 16x16x4 MFMA (operand lane l: A row / B column l % 16, k = l / 16;
+// accumulator v of lane l: column l % 16, row TailMma::row).  Gauss-Jordan by
+// pivot quads, the block pivots 2p and 2p + 1 (scalars 4p..4p+3), in the order
+// of the block form.  A step updates every entry by one rank-4 product,
 //   new = M' + A B,  A(i, k) = -col(i, k), or [i = 4p + k] on a pivot row,
 //                    B(k, j) = (Q row)(k, j), or Q(k, j - 4p) in a pivot column,
 //                    M' = M, or 0 on a pivot row or column,
 // which leaves Q (the pivot block's inverse) on the pivot block, Q row on the
-// pivot rows, -col Q in the pivot columns and M - col Q row elsewhere: two
-// MFMAs per wave.  The next quad's columns and rows, and its inverse
-// (pair_inv by lane 0 of the wave holding its pivot block, after reading the
-// block from its lanes with v_readlane), pass through LDS double buffers:
-// one barrier per step.  The columns are kept column-major and the rows
-// row-major, so that a lane writes its four consecutive column entries, and
-// reads or writes its column's four row entries, as one 16-byte access.  A
-// singular pivot block sets sing.
+// pivot rows, -col Q in the pivot columns and M - col Q row elsewhere: one
+// MFMA per accumulator.  The next quad's columns and rows pass through LDS
+// double buffers, one barrier per step.
+//
+// A step costs its longest chain and what its waves issue (4.5 cycles an
+// instruction and SIMD with four waves), so the operands reach LDS as the
+// MFMAs use them: the waves that hold the next quad write its columns negated
+// with unit pivot rows, and its rows with unit pivot columns (Q row is then Q
+// there), and clear their pivot entries right after, so no wave selects on
+// pivot rows or columns when it reads.  The next pivot block does not wait for
+// the update: wave 15 (at raised priority) forms it from LDS ahead of its own
+// tile, P' = D - col Q row on sixteen lanes, with D, the block before this
+// step, left in LDS by the step before, and inverts it through the Schur
+// complement of its first block pivot, lane r solving for row r.  Cycles a
+// step at 61 pivots: 1955 in FP32 and 3190 in FP64 (2117 and 3400 with eight
+// 32 x 64 tiles and the pivot on a wave of its own, 2419 and 3700 without the
+// priority).  One quad per step, not one block pivot, is what FP64 gains:
+// factorization of 118 buses x 200 107 -> 59 us, one 9241-bus instance 319 ->
+// 271 us; FP32, which inverted its pivot block after the update before, 48 ->
+// 42 and 196 -> 188 us.  A singular pivot block sets sing.
 constexpr int TAIL_NS = 2 * TAIL_MAX;   // scalars per side of the dense tail
+constexpr int TAIL_CS = TAIL_NS + 16;   // column stride: the four k of an A operand
+                                        // start in different LDS banks
+template <typename T>
 struct alignas(16) TailQuads {
-  float col[2][4][TAIL_NS], row[2][TAIL_NS][4], q[2][4][4];
+  T col[2][4][TAIL_CS];                 // [k][row]
+  T row[2][TAIL_NS][4];                 // [column][k]
+  T q[2][4][4];                         // the pivot block's inverse
+  T d[2][4][4];                         // the pivot block of the quad after next
 };
 
-__device__ __forceinline__ void tail_inverse_mfma(const B4<float> *D, int s, int nt,
-                                                  TailQuads &mq, B4<float> *Ti,
+template <typename T> struct TailMma;
+template <> struct TailMma<float> {
+  typedef float acc __attribute__((ext_vector_type(4)));
+  static __device__ __forceinline__ acc mma(float a, float b, acc c) {
+    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+  }
+  // row of accumulator v in lane group g = l / 16, and its inverse
+  static __device__ __forceinline__ int row(int v, int g) { return 4 * g + v; }
+};
+template <> struct TailMma<double> {
+  typedef double acc __attribute__((ext_vector_type(4)));
+  static __device__ __forceinline__ acc mma(double a, double b, acc c) {
+    return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
+  }
+  static __device__ __forceinline__ int row(int v, int g) { return g + 4 * v; }
+};
+
+__device__ __forceinline__ float lane_value(float v, int l) {
+  return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), l));
+}
+__device__ __forceinline__ double lane_value(double v, int l) {
+  const long long b = __double_as_longlong(v);
+  const unsigned lo = (unsigned)__builtin_amdgcn_readlane((int)b, l);
+  const int hi = __builtin_amdgcn_readlane((int)(b >> 32), l);
+  return __longlong_as_double(((long long)hi << 32) | lo);
+}
+
+template <typename T>
+__device__ __forceinline__ void tail_inverse_mfma(const B4<T> *D, int s, int nt,
+                                                  TailQuads<T> &mq, B4<T> *Ti,
                                                   int &sing) {
-  typedef float f32x16 __attribute__((ext_vector_type(16)));
+  typedef TailMma<T> M;
+  typedef typename M::acc Acc;
+  constexpr bool F32 = sizeof(T) == 4;
   const int n2 = 2 * s;
-  auto mget = [&](int i, int j) -> float {
+  auto mget = [&](int i, int j) -> T {
     if (i < n2 && j < n2)
       return (&D[(i >> 1) * s + (j >> 1)].a)[2 * (i & 1) + (j & 1)];
-    return i == j ? 1.f : 0.f;
+    return i == j ? (T)1 : (T)0;
   };
-  auto put_q = [&](int buf, const B4<float> (&r)[2][2]) {
-#pragma unroll
-    for (int a = 0; a < 2; a++)
-#pragma unroll
-      for (int b = 0; b < 2; b++) {
-        mq.q[buf][2 * a][2 * b] = r[a][b].a;
-        mq.q[buf][2 * a][2 * b + 1] = r[a][b].b;
-        mq.q[buf][2 * a + 1][2 * b] = r[a][b].c;
-        mq.q[buf][2 * a + 1][2 * b + 1] = r[a][b].d;
-      }
+  // row `lane` (0..3) of the inverse of the pivot block e into mq.q[buf]:
+  // with e = [[A, B], [C, E]] and S = E - C A^-1 B, the row (z1, z2) of
+  // e^-1 for the unit row (f, h) has z2 = (h - f A^-1 B) S^-1 and
+  // z1 = (f - z2 C) A^-1
+  auto invert = [&](const T (&e)[4][4], int buf, int r) {
+    const B4<T> A = {e[0][0], e[0][1], e[1][0], e[1][1]}, B = {e[0][2], e[0][3], e[1][2], e[1][3]};
+    const B4<T> C = {e[2][0], e[2][1], e[3][0], e[3][1]};
+    B4<T> S = {e[2][2], e[2][3], e[3][2], e[3][3]}, ai, si;
+    bool bad = blk_inv(A, ai);
+    const B4<T> aib = blk_mul(ai, B);
+    blk_fms(S, C, aib);
+    bad |= blk_inv(S, si);
+    if (bad) sing = 1;
+    const T f0 = r == 0 ? (T)1 : (T)0, f1 = r == 1 ? (T)1 : (T)0;
+    const T h0 = r == 2 ? (T)1 : (T)0, h1 = r == 3 ? (T)1 : (T)0;
+    const T y0 = fma(-f1, aib.c, fma(-f0, aib.a, h0)), y1 = fma(-f1, aib.d, fma(-f0, aib.b, h1));
+    const T z2 = fma(y1, si.c, y0 * si.a), z3 = fma(y1, si.d, y0 * si.b);
+    const T t0 = fma(-z3, C.c, fma(-z2, C.a, f0)), t1 = fma(-z3, C.d, fma(-z2, C.b, f1));
+    mq.q[buf][r][0] = fma(t1, ai.c, t0 * ai.a);
+    mq.q[buf][r][1] = fma(t1, ai.d, t0 * ai.b);
+    mq.q[buf][r][2] = z2;
+    mq.q[buf][r][3] = z3;
   };
   // the wave's tile in scalar registers: every choice below that depends
   // only on the tile and the step is a scalar branch
   const int lane = (int)threadIdx.x & 63;
   const int w = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
-  const int rb = (w >> 2) * 32, cb = (w & 3) * 32;
-  const int half = lane >> 5;
-  const int ia = rb + (lane & 31);   // row of the lane's A operands
-  const int jc = cb + (lane & 31);   // column of its B operands and accumulators
-  auto acc_row = [&](int v) { return rb + 8 * (v >> 2) + 4 * half + (v & 3); };
-  f32x16 acc;
+  constexpr int NR = 2, NC = 2, PIVOT_WAVE = 15;     // strips of 16 per tile
+  const int rt = (w >> 2) * NR, ct = (w & 3) * NC;   // first row / column strip
+  const int li = lane & 15, g = lane >> 4;
+  const bool tile = rt * 16 < n2 && ct * 16 < n2;  // any entry of S
+  Acc acc[NR][NC];
 #pragma unroll
-  for (int v = 0; v < 16; v++) acc[v] = mget(acc_row(v), jc);
-  if (threadIdx.x < TAIL_NS) {
-    const int q = (int)threadIdx.x;
+  for (int a = 0; a < NR; a++)
 #pragma unroll
-    for (int k = 0; k < 4; k++) {
-      mq.col[0][k][q] = mget(q, k);
-      mq.row[0][q][k] = mget(k, q);
+    for (int b = 0; b < NC; b++)
+#pragma unroll
+      for (int v = 0; v < 4; v++)
+        acc[a][b][v] = tile ? mget((rt + a) * 16 + M::row(v, g), (ct + b) * 16 + li) : (T)0;
+  // quad p's operands into LDS buffer u, its entries cleared, and the pivot
+  // block of quad p + 1; called by the waves of the tiles.  Which strip holds
+  // the quad is one scalar branch per strip (the empty asm keeps the compiler
+  // from folding it into the lanes' masks, whose bookkeeping every wave would
+  // then run for every strip).
+  auto publish = [&](int p, int u) {
+    const int ps = p >> 2, pq = p & 3, ds = (p + 1) >> 2, dq = (p + 1) & 3;
+    const bool rows = (unsigned)(ps - rt) < (unsigned)NR, cols = (unsigned)(ps - ct) < (unsigned)NC;
+    const bool lc = (li >> 2) == pq;             // the lane's column is a pivot column
+    if (rows) {
+#pragma unroll
+      for (int h = 0; h < NR; h++)
+        if (rt + h == ps) {
+          asm volatile("");
+#pragma unroll
+          for (int b = 0; b < NC; b++) {
+            T *to = mq.row[u][(ct + b) * 16 + li];
+            const bool unit = lc && ct + b == ps;
+            if (F32) {
+              if (g == pq) {
+#pragma unroll
+                for (int v = 0; v < 4; v++)
+                  to[v] = unit ? ((li & 3) == v ? (T)1 : (T)0) : acc[h][b][v];
+              }
+            } else {
+              const T x = pq == 0 ? acc[h][b][0] : pq == 1 ? acc[h][b][1]
+                        : pq == 2 ? acc[h][b][2] : acc[h][b][3];
+              to[g] = unit ? ((li & 3) == g ? (T)1 : (T)0) : x;
+            }
+          }
+        }
     }
-  }
-  if (threadIdx.x == 0) {
-    B4<float> m[2][2], r[2][2];
+    if (cols) {
 #pragma unroll
-    for (int a = 0; a < 2; a++)
+      for (int h = 0; h < NC; h++)
+        if (ct + h == ps) {
+          asm volatile("");
+          if (lc) {
 #pragma unroll
-      for (int b = 0; b < 2; b++)
-        m[a][b] = {mget(2 * a, 2 * b), mget(2 * a, 2 * b + 1),
-                   mget(2 * a + 1, 2 * b), mget(2 * a + 1, 2 * b + 1)};
-    if (pair_inv(m, r)) sing = 1;
-    put_q(0, r);
+            for (int a = 0; a < NR; a++)
+#pragma unroll
+              for (int v = 0; v < 4; v++) {
+                const int i = M::row(v, g);
+                const bool unit = (i >> 2) == pq && rt + a == ps;
+                mq.col[u][li & 3][(rt + a) * 16 + i] =
+                    unit ? ((i & 3) == (li & 3) ? (T)1 : (T)0) : -acc[a][h][v];
+                acc[a][h][v] = (T)0;
+              }
+          }
+        }
+    }
+    if ((unsigned)(ds - rt) < (unsigned)NR && (unsigned)(ds - ct) < (unsigned)NC) {
+#pragma unroll
+      for (int a = 0; a < NR; a++)               // the block of quad p + 1
+#pragma unroll
+        for (int h = 0; h < NC; h++)
+          if (rt + a == ds && ct + h == ds) {
+            asm volatile("");
+            if ((li >> 2) == dq) {
+#pragma unroll
+              for (int v = 0; v < 4; v++)
+                if ((M::row(v, g) >> 2) == dq) mq.d[u][M::row(v, g) & 3][li & 3] = acc[a][h][v];
+            }
+          }
+    }
+    if (rows) {
+#pragma unroll
+      for (int h = 0; h < NR; h++)
+        if (rt + h == ps) {
+          asm volatile("");
+#pragma unroll
+          for (int b = 0; b < NC; b++)
+#pragma unroll
+            for (int v = 0; v < 4; v++)
+              if ((M::row(v, g) >> 2) == pq) acc[h][b][v] = (T)0;
+        }
+    }
+  };
+  if (w == PIVOT_WAVE && lane < 4) {
+    T e[4][4];
+#pragma unroll
+    for (int a = 0; a < 4; a++)
+#pragma unroll
+      for (int b = 0; b < 4; b++) e[a][b] = mget(a, b);
+    invert(e, 0, lane);
   }
+  if (tile) publish(0, 0);
+  if (w == PIVOT_WAVE) __builtin_amdgcn_s_setprio(3);
   __syncthreads();
   for (int p = 0; p < nt; p++) {
     const int cur = p & 1, nxt = cur ^ 1;
-    const bool prow = (ia >> 2) == p, pcol = (jc >> 2) == p;
-    float a[2], b[2];
+    if (w == PIVOT_WAVE && p + 1 < nt) {
+      // the next pivot block, lane 4 a + b its entry (a, b), and its inverse
+      const int a = (lane >> 2) & 3, b = lane & 3, nb = 4 * (p + 1);
+      T r[4], pe = mq.d[cur][a][b];
 #pragma unroll
-    for (int h = 0; h < 2; h++) {
-      const int k = 2 * h + half;
-      a[h] = prow ? ((ia & 3) == k ? 1.f : 0.f) : -mq.col[cur][k][ia];
-      const float4 rw = *(const float4 *)mq.row[cur][jc];
-      const float4 qk = *(const float4 *)mq.q[cur][k];
-      const float qr = qk.x * rw.x + qk.y * rw.y + qk.z * rw.z + qk.w * rw.w;
-      b[h] = pcol ? mq.q[cur][k][jc & 3] : qr;
+      for (int m = 0; m < 4; m++) r[m] = mq.row[cur][nb + b][m];
+#pragma unroll
+      for (int k = 0; k < 4; k++) {
+        T y = mq.q[cur][k][0] * r[0];
+#pragma unroll
+        for (int m = 1; m < 4; m++) y = fma(mq.q[cur][k][m], r[m], y);
+        pe = fma(mq.col[cur][k][nb + a], y, pe);
+      }
+      T e[4][4];
+#pragma unroll
+      for (int k = 0; k < 4; k++)
+#pragma unroll
+        for (int m = 0; m < 4; m++) e[k][m] = lane_value(pe, 4 * k + m);
+      if (lane < 4) invert(e, nxt, lane);
     }
+    if (tile) {
+      T av[NR], bv[NC], qk[4], rw[NC][4];
 #pragma unroll
-    for (int v = 0; v < 16; v++)
-      if (pcol || (acc_row(v) >> 2) == p) acc[v] = 0.f;
-    acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a[0], b[0], acc, 0, 0, 0);
-    acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a[1], b[1], acc, 0, 0, 0);
-    if (p + 1 < nt) {
-      const int nb = 4 * (p + 1);
-      if (nb >= rb && nb < rb + 32) {   // the next quad's rows
-        const int qq = (nb - rb) >> 2, g = qq >> 1;
-        float rv[4];
-        if (g == 0) {
+      for (int h = 0; h < NR; h++) av[h] = mq.col[cur][g][(rt + h) * 16 + li];
 #pragma unroll
-          for (int k = 0; k < 4; k++) rv[k] = acc[k];
-        } else if (g == 1) {
+      for (int k = 0; k < 4; k++) qk[k] = mq.q[cur][g][k];
 #pragma unroll
-          for (int k = 0; k < 4; k++) rv[k] = acc[4 + k];
-        } else if (g == 2) {
+      for (int h = 0; h < NC; h++)
 #pragma unroll
-          for (int k = 0; k < 4; k++) rv[k] = acc[8 + k];
-        } else {
+        for (int k = 0; k < 4; k++) rw[h][k] = mq.row[cur][(ct + h) * 16 + li][k];
 #pragma unroll
-          for (int k = 0; k < 4; k++) rv[k] = acc[12 + k];
-        }
-        if (half == (qq & 1))
-          *(float4 *)mq.row[nxt][jc] = make_float4(rv[0], rv[1], rv[2], rv[3]);
-        if (nb >= cb && nb < cb + 32) {   // and its pivot block
-          const int src = 32 * (qq & 1) + (nb - cb);   // the same in every lane
-          float e[4][4];
+      for (int h = 0; h < NC; h++)
+        bv[h] = fma(qk[3], rw[h][3], fma(qk[2], rw[h][2], fma(qk[1], rw[h][1], qk[0] * rw[h][0])));
 #pragma unroll
-          for (int k = 0; k < 4; k++)
+      for (int b = 0; b < NC; b++)
 #pragma unroll
-            for (int m = 0; m < 4; m++)
-              e[k][m] = __int_as_float(
-                  __builtin_amdgcn_readlane(__float_as_int(rv[k]), src + m));
-          if (lane == 0) {
-            B4<float> m[2][2], r[2][2];
-#pragma unroll
-            for (int x = 0; x < 2; x++)
-#pragma unroll
-              for (int y = 0; y < 2; y++)
-                m[x][y] = {e[2 * x][2 * y], e[2 * x][2 * y + 1], e[2 * x + 1][2 * y],
-                           e[2 * x + 1][2 * y + 1]};
-            if (pair_inv(m, r)) sing = 1;
-            put_q(nxt, r);
-          }
-        }
-      }
-      if (nb >= cb && nb < cb + 32) {   // the next quad's columns
-        const int k = (lane & 31) - (nb - cb);
-        if (k >= 0 && k < 4)
-#pragma unroll
-          for (int v = 0; v < 16; v += 4)
-            *(float4 *)&mq.col[nxt][k][acc_row(v)] =
-                make_float4(acc[v], acc[v + 1], acc[v + 2], acc[v + 3]);
-      }
+        for (int a = 0; a < NR; a++) acc[a][b] = M::mma(av[a], bv[b], acc[a][b]);
+      if (p + 1 < nt) publish(p + 1, nxt);
     }
     __syncthreads();
   }
+  if (w == PIVOT_WAVE) __builtin_amdgcn_s_setprio(0);
+  if (tile) {
 #pragma unroll
-  for (int v = 0; v < 16; v++) {
-    const int i = acc_row(v);
-    if (i < n2 && jc < n2) (&Ti[(i >> 1) * s + (jc >> 1)].a)[2 * (i & 1) + (jc & 1)] = acc[v];
+    for (int a = 0; a < NR; a++)
+#pragma unroll
+      for (int b = 0; b < NC; b++)
+#pragma unroll
+        for (int v = 0; v < 4; v++) {
+          const int i = (rt + a) * 16 + M::row(v, g), j = (ct + b) * 16 + li;
+          if (i < n2 && j < n2)
+            (&Ti[(i >> 1) * s + (j >> 1)].a)[2 * (i & 1) + (j & 1)] = acc[a][b][v];
+        }
   }
 }
 
@@ -1026,7 +1137,7 @@ __global__ void k_jacobian(DevTopo g, DevInst d, B4<T> *LU, int elim0, int rhs) 
 // complement S = A_SS - L_SN U_NS is assembled in LDS and inverted in place
 // by Gauss-Jordan with the same pivot order (one barrier per step: the next
 // pivot rows, columns and inverse are captured into double buffers while
-// the current step updates): FP32 on 1024 lanes by pivot quads on the matrix
+// the current step updates): on 1024 lanes by pivot quads on the matrix
 // cores (tail_inverse_mfma), otherwise by pivot pairs (FP32) or single
 // pivots (FP64) on the vector ALUs; S^-1 goes to TL for the sweeps.
 // ---------------------------------------------------------------------------
@@ -1081,7 +1192,7 @@ __device__ __forceinline__ void lu_factor_body(DevTopo g, InstState *st, int cou
     } gj;
     // the same on matrix cores, in scalars: the next pivot quad's columns,
     // rows and inverse
-    TailQuads mq;
+    TailQuads<T> mq;
   };
   __shared__ TabStage sh;
   int4 *const s_ch = sh.tab.ch;
@@ -1381,8 +1492,8 @@ __device__ __forceinline__ void lu_factor_body(DevTopo g, InstState *st, int cou
     // 2x2 tiles of blocks per side; an odd size gets an identity pivot
     // appended (zero coupling: every other value comes out unchanged)
     const int se = s + (s & 1), nt = se / 2;
-    if (sizeof(T) == 4 && P.tail_mfma && blockDim.x == 1024) {
-      if constexpr (sizeof(T) == 4) tail_inverse_mfma(D, s, nt, sh.mq, Ti, sing);
+    if (P.tail_mfma && blockDim.x == 1024) {
+      tail_inverse_mfma<T>(D, s, nt, sh.mq, Ti, sing);
     } else if (sizeof(T) == 4 && nt * nt <= (int)blockDim.x) {
       // FP32: Gauss-Jordan by pivot pairs, each thread owning a 2x2 tile for
       // the whole elimination: per step the pair's inverse Q (formed by the
