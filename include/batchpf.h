@@ -430,7 +430,9 @@ bpf_status bpf_set_launch(bpf_engine *e, int32_t lu_threads,
 /* Run-time schedule choices (the autotuner sets them; 0 keeps the current
  * value): newton_per_graph = Newton iterations per captured graph (1..16;
  * the host reads the active-instance counts once per round of replays);
- * tail_inverse = 1 matrix cores, 2 vector ALUs (FP32 dense-tail inverse);
+ * tail_inverse = 1 matrix cores, 2 vector ALUs (dense-tail inverse; with 1 and
+ * 1024 factorization lanes the levels below the tail run from LDS in parts,
+ * otherwise in chunks of products);
  * sweep_form = 1 slot form, 2 entry-parallel, 3 level rows (the first that
  * applies, in that order, from the chosen one); parts = 1..4: the Newton
  * loop runs the batch as that many parts of consecutive instances, each on
@@ -451,15 +453,17 @@ bpf_status bpf_set_schedule(bpf_engine *e, int32_t newton_per_graph,
  * with active instances x workgroups within the compute units of the
  * batch's part); 1: never; 2, 4, 8: always that many where the analysis
  * planned them.  Results do not depend on it: every output is summed in
- * the same order. */
+ * the same order.  It concerns the factorization in chunks; the one from LDS
+ * gives every part a workgroup at any count. */
 bpf_status bpf_set_factor_split(bpf_engine *e, int32_t workgroups);
 
 /* Forward substitution inside the factorization (no counterpart in the
  * reference, whose solves run both sweeps): while at most `max_active`
  * instances of a batch part are active, the Newton step's factorization
  * also forms L^-1 of the mismatch and the first solve skips its forward
- * sweep; above that both run as usual (-1: never; default 32).  Only the
- * slot-form sweeps use it.  Results agree to rounding either way. */
+ * sweep; above that both run as usual (-1: never; default 32 for the
+ * factorization in chunks, no limit for the one from LDS, which carries the
+ * right-hand side as one more row).  Only the slot-form sweeps use it.  Results agree to rounding either way. */
 bpf_status bpf_set_fused_forward(bpf_engine *e, int32_t max_active);
 
 #ifdef __cplusplus

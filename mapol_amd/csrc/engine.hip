@@ -18,6 +18,7 @@
 
 #include "../../include/batchpf.h"
 #include "kernels.hip"
+#include "resident.hip"
 #include "symbolic.hpp"
 
 using namespace bpf;
@@ -109,7 +110,13 @@ struct bpf_engine {
   // Newton factors are FP32 (so that neither disturbs the Newton buffers or
   // the captured graph), and the adjoint's per-instance arrays; allocated on
   // first use for the current instance count
-  struct Fp64Factors { void *LU = nullptr, *TL = nullptr, *xglob = nullptr; } f64;
+  struct Fp64Factors { void *LU = nullptr, *TL = nullptr, *xglob = nullptr, *UPD = nullptr; } f64;
+  // LDS-resident factorization, per precision (0 FP32: mixed Newton steps, 1
+  // FP64): the plan, its first part of each stage (empty: the tree does not
+  // fit it), and the Newton factors' updates between parts [T][2 * nupd]
+  ResPlan res[2]{};
+  std::vector<int> res_stage[2];
+  void *d_UPD = nullptr;
   struct AdjBufs {
     double *rate = nullptr, *G = nullptr, *lam = nullptr, *gP = nullptr,
            *gQ = nullptr, *gx = nullptr, *obj = nullptr;
@@ -153,6 +160,7 @@ struct bpf_engine {
   // the compute units and the parts running side by side set the budget
   bool fplan_split = false;
   int split_mode = 0;
+  bool fused_set = false;            // bpf_set_fused_forward was called
   int num_cu = 256;
   int parts_running = 1;
   bool capturing = false;            // recording the iteration graph
@@ -327,6 +335,43 @@ static bpf_status bus_rows_upload(bpf_engine *e, const cd *src, cd *ddst, size_t
                      (const cd *)e->d_bus_stage, ddst, e->d_bus_ext, e->n, (int)T);
   HIPCHK(hipGetLastError());
   HIPCHK(hipStreamSynchronize(e->stream));
+  return BPF_OK;
+}
+
+// the LDS-resident plan of one precision, uploaded as one buffer
+static bpf_status build_resident_plan(bpf_engine *e, int fp64) {
+  ResidentPlan H;
+  const int sc = fp64 ? 8 : 4;
+  build_resident(e->S, resident_cap(RES_TOP_LDS, sc), resident_cap(RES_SMALL_LDS, sc), H);
+  if (!H.ok) return BPF_OK;
+  ResPlan &R = e->res[fp64];
+  const std::vector<int> word(H.word.begin(), H.word.end()), desc(H.desc.begin(), H.desc.end());
+  const std::vector<int> *src[] = {&H.part, &H.wave, &H.slot_pos, &H.upd_ptr, &H.upd, &word,
+                                   &desc, &H.tail, &H.tail_ptr, &H.tail_upd};
+  std::vector<int> all;
+  size_t at[10];
+  for (int k = 0; k < 10; k++) {
+    at[k] = all.size();
+    all.insert(all.end(), src[k]->begin(), src[k]->end());
+    all.resize((all.size() + 4 + 31) / 32 * 32, 0);   // never empty, 128-byte aligned
+  }
+  const int *p;
+  bpf_status s = upload(e, e->owned, all, &p);
+  if (s) return s;
+  R.part = (const int4 *)(p + at[0]);
+  R.wave = (const int4 *)(p + at[1]);
+  R.slot_pos = (const int2 *)(p + at[2]);
+  R.upd_ptr = p + at[3];
+  R.upd = p + at[4];
+  R.word = (const unsigned *)(p + at[5]);
+  R.desc = (const unsigned *)(p + at[6]);
+  R.tail = (const int4 *)(p + at[7]);
+  R.tail_ptr = p + at[8];
+  R.tail_upd = p + at[9];
+  R.nupd = H.nupd;
+  R.tn = e->S.tail_n;
+  R.ntail = (int)H.tail.size() / 4;
+  e->res_stage[fp64] = H.stage;
   return BPF_OK;
 }
 
@@ -670,6 +715,8 @@ extern "C" bpf_status bpf_create(const bpf_case *c, const bpf_options *o,
     SP.sl_nfw_t = S.sl_nfw_t;
     SP.sl_nbw_t = S.sl_nbw_t;
   }
+  if ((s = build_resident_plan(e, 1))) return s;
+  if (e->opt.precision == BPF_MIXED && (s = build_resident_plan(e, 0))) return s;
   e->sweep_form = 0;
   e->tail_form = BPF_TAIL_MFMA;
 #undef UP
@@ -709,6 +756,7 @@ extern "C" bpf_status bpf_set_fused_forward(bpf_engine *e, int32_t max_active) {
     e->err = "fused forward substitution: -1 (never) or the most active instances";
     return BPF_ERR_INVALID_ARG;
   }
+  e->fused_set = true;
   e->fplan.fused_limit = max_active;
   e->splan.fused_limit = max_active;
   drop_graphs(e);
@@ -769,7 +817,7 @@ extern "C" bpf_status bpf_set_instances(bpf_engine *e, int32_t T,
     // the factor storage lived in that pool too: forget it, so that
     // ensure_lu allocates it for the new T instead of freeing the stale
     // address again (which a new buffer of this call may have been given)
-    e->d_LU = e->d_xglob = e->d_TL = nullptr;
+    e->d_LU = e->d_xglob = e->d_TL = e->d_UPD = nullptr;
     e->f64 = bpf_engine::Fp64Factors();
     e->adj = bpf_engine::AdjBufs();
     e->lu_fp64 = -1;
@@ -866,6 +914,7 @@ extern "C" bpf_status bpf_set_instances(bpf_engine *e, int32_t T,
 // (re)allocate the factor storage for the requested precision
 static bpf_status ensure_lu(bpf_engine *e, int fp64) {
   if (e->lu_fp64 == fp64 && e->d_LU) return BPF_OK;
+  bpf_status s;
   if (e->d_LU) {
     for (auto it = e->inst_owned.begin(); it != e->inst_owned.end(); ++it)
       if (it->p == e->d_LU) { hipFree(it->p); e->inst_owned.erase(it); break; }
@@ -873,10 +922,14 @@ static bpf_status ensure_lu(bpf_engine *e, int fp64) {
       if (it->p == e->d_xglob) { hipFree(it->p); e->inst_owned.erase(it); break; }
     for (auto it = e->inst_owned.begin(); it != e->inst_owned.end(); ++it)
       if (it->p == e->d_TL) { hipFree(it->p); e->inst_owned.erase(it); break; }
-    e->d_LU = e->d_xglob = e->d_TL = nullptr;
+    for (auto it = e->inst_owned.begin(); it != e->inst_owned.end(); ++it)
+      if (it->p == e->d_UPD) { hipFree(it->p); e->inst_owned.erase(it); break; }
+    e->d_LU = e->d_xglob = e->d_TL = e->d_UPD = nullptr;
   }
   size_t el = fp64 ? sizeof(B4<double>) : sizeof(B4<float>);
-  bpf_status s = dalloc(e, e->inst_owned, el * (size_t)e->T * e->g.nnzLU, &e->d_LU);
+  s = dalloc(e, e->inst_owned, el * (size_t)e->T * e->g.nnzLU, &e->d_LU);
+  if (s) return s;
+  s = dalloc(e, e->inst_owned, el * (size_t)e->T * 2 * e->res[fp64].nupd, &e->d_UPD);
   if (s) return s;
   s = dalloc(e, e->inst_owned, el * (size_t)e->T * e->S.tail_n * e->S.tail_n,
              &e->d_TL);
@@ -909,6 +962,7 @@ static bpf_status fp64_factors(bpf_engine *e, B4<double> **LU, B4<double> **TL,
     bpf_status s = dalloc(e, e->inst_owned, el * (size_t)e->T * e->g.nnzLU, &f.LU);
     if (!s) s = dalloc(e, e->inst_owned,
                        el * (size_t)e->T * e->S.tail_n * e->S.tail_n, &f.TL);
+    if (!s) s = dalloc(e, e->inst_owned, el * (size_t)e->T * 2 * e->res[1].nupd, &f.UPD);
     const size_t xs = sizeof(double) * 2 * (size_t)e->S.nb;
     if (!s && xs > (size_t)SOLVE_LDS_BYTES)
       s = dalloc(e, e->inst_owned, xs * e->T, &f.xglob);
@@ -998,10 +1052,12 @@ static void launch_solve(bpf_engine *e, int T_, const void *LU, int rhs_mode,
                          const void *TL = nullptr, void *xglob = nullptr) {
   const int th = e->solve_threads;
   if (!TL) { TL = e->d_TL; xglob = e->d_xglob; }
+  SolvePlan sp_ = e->splan;
+  sp_.fused_limit = e->fused_forward;     // as the factorization of this step
   auto go = [&](auto kern) {
     hipLaunchKernelGGL(kern, dim3(T_), dim3(th), 0, e->stream, e->g, e->d,
                        (const B4<T> *)LU, (const B4<T> *)TL, rhs_mode,
-                       accumulate, e->splan, use_lds, ep, (T *)xglob);
+                       accumulate, sp_, use_lds, ep, (T *)xglob);
   };
   const int sp = slot_lanes(e, ep);
   if (sp > 0) {
@@ -1012,6 +1068,41 @@ static void launch_solve(bpf_engine *e, int T_, const void *LU, int rhs_mode,
   } else {
     go(k_lu_solve<T, 0>);
   }
+}
+
+// the LDS-resident form of the factorization (1024 lanes, tail on the matrix
+// cores); the other launch shapes and the vector-ALU tail keep the chunks
+static bool resident_runs(const bpf_engine *e, int fp64) {
+  return !e->res_stage[fp64].empty() && e->lu_threads == RES_TOP_LANES &&
+         e->fplan.tail_mfma;
+}
+
+// every part of a stage and instance its own workgroup, one launch a stage;
+// l0: level 0 was finished by the Jacobian fill
+template <typename T>
+static void launch_resident(bpf_engine *e, B4<T> *LU, B4<T> *TL, B4<T> *UPD, int l0,
+                            int count_iter) {
+  const int fp64 = sizeof(T) == 8;
+  const ResPlan &R = e->res[fp64];
+  const std::vector<int> &sg = e->res_stage[fp64];
+  const int last = (int)sg.size() - 2;
+  for (int q = 0; q < last; q++)
+    hipLaunchKernelGGL(k_res_parts<T>, dim3((unsigned)e->T * (sg[q + 1] - sg[q])),
+                       dim3(RES_SMALL_LANES), 0, e->stream, e->g, (const InstState *)e->d.st, R,
+                       sg[q], sg[q + 1] - sg[q], l0, q > 0 ? 1 : 0, LU, UPD, e->d.jsing);
+  hipLaunchKernelGGL(k_res_top<T>, dim3(e->T), dim3(RES_TOP_LANES), 0, e->stream, e->g, e->d.st,
+                     count_iter, R, sg[last], l0, last > 0 ? 1 : 0, LU, TL, UPD, e->d.jsing);
+}
+
+// FP64 factorization outside the Newton step (level 0 included)
+static void factor_fp64(bpf_engine *e, B4<double> *LU, B4<double> *TL) {
+  if (resident_runs(e, 1)) {
+    B4<double> *UPD = (B4<double> *)(e->opt.precision == BPF_FP64 ? e->d_UPD : e->f64.UPD);
+    launch_resident<double>(e, LU, TL, UPD, 0, 0);
+    return;
+  }
+  hipLaunchKernelGGL(k_lu_factor<double>, dim3(e->T), dim3(e->lu_threads), 0, e->stream,
+                     e->g, e->d.st, 0, e->fplan, LU, TL, 0, e->d.jsing, 0, nullptr, 0, -1);
 }
 
 template <typename T>
@@ -1029,6 +1120,10 @@ static void launch_newton_step(bpf_engine *e) {
   const int fused = slot_lanes(e, ep) > 0 && e->fplan.fused_limit >= 0 ? 1 : 0;
   FactorPlan fp = e->fplan;
   if (!fused) fp.fused_limit = -1;
+  const bool resident = resident_runs(e, sizeof(T) == 8);
+  // resident parts carry the right-hand side as one more row of their slots,
+  // whatever the active count, so the limit is the caller's or none
+  if (resident && fused && !e->fused_set) fp.fused_limit = 1 << 20;
   e->fused_forward = fused ? fp.fused_limit : -1;
   tbegin(e, "jacobian");
   hipLaunchKernelGGL(k_jacobian<T>, xgrid(e->T, ((size_t)e->g.nJb + 1) / 2, 256),
@@ -1036,7 +1131,9 @@ static void launch_newton_step(bpf_engine *e) {
                      fp.fused_limit);
   tend(e);
   tbegin(e, "lu_factor");
-  if (e->split_mode != 1 && e->fplan_split) {
+  if (resident) {
+    launch_resident<T>(e, LU, (B4<T> *)e->d_TL, (B4<T> *)e->d_UPD, c0 > 0 ? 1 : 0, 1);
+  } else if (e->split_mode != 1 && e->fplan_split) {
     // split launch pair: the subtrees below the cut with several workgroups
     // per instance when few instances are active, then the top; the
     // workgroup count follows the batch's active-instance counter (the
@@ -1100,7 +1197,7 @@ static void launch_iteration(bpf_engine *e) {
 struct PartView {
   DevInst d;
   int T;
-  void *LU, *TL, *xg;
+  void *LU, *TL, *xg, *UPD;
   hipStream_t s;
   int *hc;
 };
@@ -1125,6 +1222,7 @@ static PartView part_view(bpf_engine *e, int h, int K) {
   const size_t tn = e->S.tail_n;
   v.LU = (char *)e->d_LU + o * el * e->g.nnzLU;
   v.TL = (char *)e->d_TL + o * el * tn * tn;
+  v.UPD = (char *)e->d_UPD + o * el * 2 * e->res[e->lu_fp64 == 1].nupd;
   v.xg = e->d_xglob ? (char *)e->d_xglob + o * (e->lu_fp64 ? 8 : 4) * nb2 : nullptr;
   v.s = h == 0 ? e->stream : e->sub[h];
   v.hc = e->h_count + h;
@@ -1137,17 +1235,19 @@ struct PartScope {
   bpf_engine *e;
   DevInst d;
   int T;
-  void *LU, *TL, *xg;
+  void *LU, *TL, *xg, *UPD;
   hipStream_t s;
   int *hc;
   PartScope(bpf_engine *e_, const PartView &v)
       : e(e_), d(e_->d), T(e_->T), LU(e_->d_LU), TL(e_->d_TL), xg(e_->d_xglob),
-        s(e_->stream), hc(e_->h_count) {
+        UPD(e_->d_UPD), s(e_->stream), hc(e_->h_count) {
     e->d = v.d; e->T = v.T; e->d_LU = v.LU; e->d_TL = v.TL; e->d_xglob = v.xg;
+    e->d_UPD = v.UPD;
     e->stream = v.s; e->h_count = v.hc;
   }
   ~PartScope() {
     e->d = d; e->T = T; e->d_LU = LU; e->d_TL = TL; e->d_xglob = xg;
+    e->d_UPD = UPD;
     e->stream = s; e->h_count = hc;
   }
 };
@@ -1284,8 +1384,7 @@ static bpf_status run_fd(bpf_engine *e) {
                      e->stream, e->g, e->d, e->opt.alg, LU);
   tend(e);
   tbegin(e, "lu_factor");
-  hipLaunchKernelGGL(k_lu_factor<double>, dim3(T), dim3(e->lu_threads), 0,
-                     e->stream, e->g, e->d.st, 0, e->fplan, LU, TLd, 0, e->d.jsing, 0, nullptr, 0, -1);
+  factor_fp64(e, LU, TLd);
   tend(e);
   size_t xs = sizeof(double) * 2 * (size_t)e->S.nb;
   int use_lds = xs <= (size_t)SOLVE_LDS_BYTES;
@@ -1948,8 +2047,7 @@ extern "C" bpf_status bpf_adjoint(bpf_engine *e, const double *rate, double w,
   tbegin(e, "adjoint");
   hipLaunchKernelGGL(k_jacobian<double>, xgrid(TT, ((size_t)e->g.nJb + 1) / 2, 256),
                      dim3(256), 0, e->stream, e->g, e->d, LU, 0, -1);
-  hipLaunchKernelGGL(k_lu_factor<double>, dim3(TT), dim3(e->lu_threads), 0,
-                     e->stream, e->g, e->d.st, 0, e->fplan, LU, TLd, 0, e->d.jsing, 0, nullptr, 0, -1);
+  factor_fp64(e, LU, TLd);
   hipLaunchKernelGGL(k_adj_rhs, dim3(div_up(e->S.nb, 256), TT), dim3(256), 0,
                      e->stream, e->g, e->d, d_rate, w, a.G);
   size_t xs = sizeof(double) * nb2;
@@ -2092,8 +2190,7 @@ extern "C" bpf_status bpf_stage_fd_halfstep(bpf_engine *e, const double *V,
   // the angle (P) or magnitude (Q) update: the body of fdpf.h:480-560
   hipLaunchKernelGGL(k_bmat, dim3(div_up(e->g.nnzY, 256), T), dim3(256), 0,
                      e->stream, e->g, e->d, e->opt.alg, LU);
-  hipLaunchKernelGGL(k_lu_factor<double>, dim3(T), dim3(e->lu_threads), 0,
-                     e->stream, e->g, e->d.st, 0, e->fplan, LU, TLd, 0, e->d.jsing, 0, nullptr, 0, -1);
+  factor_fp64(e, LU, TLd);
   mismatch_pair(e, 2, e->opt.maxit_fd, 0, 1);
   const size_t xs = sizeof(double) * 2 * (size_t)e->S.nb;
   const int use_lds = xs <= (size_t)SOLVE_LDS_BYTES;

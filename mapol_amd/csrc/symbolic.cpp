@@ -634,6 +634,7 @@ bool analyse(int n, int m, const int *from, const int *to, const int *type,
   // (an L output also reduces its pivot's products; ties keep the order of
   // pks), then their products in task order.  Appends to the three lists;
   // returns {tasks, longest reduction}.
+  std::vector<int> piv_start(nb, 0);
   int rhs_out[2] = {0, 0};   // the last chunk's forward-substitution outputs, products
   auto emit_chunk = [&](const std::vector<int> &pks, std::vector<int> &tk_a,
                         std::vector<int> &tk_b, std::vector<int> &prs) {
@@ -662,17 +663,19 @@ bool analyse(int n, int m, const int *from, const int *to, const int *type,
                        if (rhs_task(x) != rhs_task(y)) return rhs_task(y);
                        return work(x) > work(y);
                      });
-    // pair offsets of every task (in chunk order)
-    std::map<std::pair<int, int>, int> start;
+    // the pivots' pair offsets (tasks take their pairs in chunk order)
     int off = (int)prs.size() / 2;
-    for (auto &x : ord) { start[x] = off; off += (int)pgroup[x.first][x.second].L.size(); }
+    for (auto &x : ord) {
+      if (x.second == 0) piv_start[x.first] = off;
+      off += (int)pgroup[x.first][x.second].L.size();
+    }
     int wmax = 0;
     for (auto &x : ord) {
       const Task &t = pgroup[x.first][x.second];
-      const int p0 = start[x], p1 = p0 + (int)t.L.size();
+      const int p0 = (int)prs.size() / 2, p1 = p0 + (int)t.L.size();
       tk_a.insert(tk_a.end(), {t.dst, p0, p1, 0});
       if (t.dst & TASK_LCOL) {
-        const int v0 = start[{x.first, 0}], v1 = v0 + (int)pgroup[x.first][0].L.size();
+        const int v0 = piv_start[x.first], v1 = v0 + (int)pgroup[x.first][0].L.size();
         tk_b.insert(tk_b.end(), {0, v0, v1, 0});
       } else {
         tk_b.insert(tk_b.end(), {0, 0, 0, 0});

@@ -610,7 +610,8 @@ class Engine:
     def set_fused_forward(self, max_active=32):
         """the Newton step's factorization forms the forward substitution
         (and the first solve skips its forward sweep) while at most
-        ``max_active`` instances of a batch part are active; -1 never
+        ``max_active`` instances of a batch part are active; -1 never, no
+        limit where this is not called and the factorization runs from LDS
         (``bpf_set_fused_forward``)"""
         self._check(self.L.bpf_set_fused_forward(self.h, int(max_active)),
                     "bpf_set_fused_forward")
