@@ -2058,10 +2058,10 @@ extern "C" bpf_status bpf_adjoint(bpf_engine *e, const double *rate, double w,
   const int th = e->solve_threads;
   if (e->S.sl_ok_t &&
       sweep_mode(e->S, sizeof(double), use_lds, e->sweep_form, 512) == 2) {
-    hipLaunchKernelGGL(k_adj_solve_slot<SLOT_CHUNK / 512>, dim3(TT), dim3(512), 0,
-                       e->stream, e->g, e->d, (const B4<double> *)LU,
-                       (const B4<double> *)TLd, (const double *)a.G, a.lam,
-                       e->splan);
+    hipLaunchKernelGGL(e->S.prm.slot_chunk <= 1024 ? k_adj_solve_slot<2> : k_adj_solve_slot<4>,
+                       dim3(TT), dim3(512), 0, e->stream, e->g, e->d,
+                       (const B4<double> *)LU, (const B4<double> *)TLd,
+                       (const double *)a.G, a.lam, e->splan);
   } else {
     hipLaunchKernelGGL(k_adj_solve, dim3(TT), dim3(th),
                        0, e->stream, e->g, e->d, (const B4<double> *)LU,

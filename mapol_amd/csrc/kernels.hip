@@ -2081,9 +2081,13 @@ __device__ __forceinline__ void lu_sweeps_ep(const B4<T> *A, const B4<T> *Ti,
 // reads beyond), and that lane updates x_i (backward: times the pivot
 // inverse).  One barrier per chunk.  Loads run two stages ahead as in the
 // entry-parallel form (slot descriptors two chunks ahead, factor blocks one
-// chunk ahead); a wave skips the slot blocks it has no lane in with a scalar
-// branch, so load counts vary and one explicit wait at the top of each chunk
-// receives everything the previous chunk requested.
+// chunk ahead); one explicit wait at the top of each chunk receives everything
+// the previous chunk requested.
+// Bound by what the waves issue: most chunks fill one to four waves, so the
+// chunk's range sits in scalar registers (lanes hold 64 ranges, read with
+// v_readlane) and a wave without slots goes through its tests and the barrier
+// only.  A mixed-precision pass, 9241 buses: one instance 82 -> 69 us, 200
+// instances 116 -> 104; in FP64 117 -> 69 and 184 -> 123 (with SLOT_LANES).
 // sum of the lanes of each aligned group of 2^lg lanes into the group's
 // first lane.  An unconditional tree (step s: lane i adds lane i + 2^s) leaves
 // in the first lane of every aligned window of 2^(s+1) lanes that window's
@@ -2153,113 +2157,91 @@ struct SlotVal {
   B4<T> d[SP];      // pivot inverses (backward sweep, groups' first lanes)
 };
 
-// The slot descriptors are loaded by every wave (clamped to the chunk's last
-// slot): a load that a wave may skip leaves the register's previous value
-// on the skipping path, and the compiler waits for the load before merging
-// the two.  The blocks are loaded only by waves with a slot in the block
-// (their registers are not read otherwise, so nothing merges).
+// a wave's share of chunk range [x, y): its slots k * lanes + 64 wave ..; a
+// chunk spans whole 64-slot windows, so a wave has all 64 slots or none
+__device__ __forceinline__ bool slot_on(int2 m, int wv, int k) {
+  return m.x + 64 * wv + k * (int)blockDim.x < m.y;
+}
+
 template <int SP>
-__device__ __forceinline__ SlotIdx<SP> slot_index(const int4 *slot, const int4 &m) {
-  SlotIdx<SP> ix;
+__device__ __forceinline__ void slot_index(const int4 *slot, int2 m, int wv, SlotIdx<SP> &ix) {
 #pragma unroll
-  for (int k = 0; k < SP; k++) {
-    const int q = m.x + (int)threadIdx.x + k * (int)blockDim.x;
-    ix.s[k] = slot[min(q, m.y - 1)];
-  }
-  return ix;
+  for (int k = 0; k < SP; k++)
+    if (slot_on(m, wv, k)) ix.s[k] = slot[m.x + (int)threadIdx.x + k * (int)blockDim.x];
 }
 
 // TR: the transposed sweeps (U^T forward with the pivots, L^T backward),
 // whose slots hold mirror positions; the pivots then belong to the forward
 // chunks
-template <typename T, int SP, bool TR = false>
-__device__ __forceinline__ SlotVal<T, SP> slot_values(const B4<T> *A,
-                                                      const int4 &m, bool bw,
-                                                      const SlotIdx<SP> &ix) {
-  SlotVal<T, SP> v;
+template <typename T, int SP, bool TR>
+__device__ __forceinline__ void slot_values(const B4<T> *A, int2 m, int wv, bool bw,
+                                            const SlotIdx<SP> &ix, SlotVal<T, SP> &v) {
   const bool piv = TR ? !bw : bw;
 #pragma unroll
-  for (int k = 0; k < SP; k++) {
-    const int q = m.x + (int)threadIdx.x + k * (int)blockDim.x;
-    if (wave_any(q, m.y)) {
+  for (int k = 0; k < SP; k++)
+    if (slot_on(m, wv, k)) {
       v.a[k] = A[pinned(ix.s[k].x)];
       if (piv) v.d[k] = A[pinned(ix.s[k].w)];
     }
-  }
-  return v;
 }
 
-// chunk c (range m; slots cur, blocks val, both received): the ranges of
-// chunks c + 1 (mn) and c + 2 (ma) are read first, then every x the chunk
-// needs; while those reads are in flight the blocks of chunk c + 1 are
-// requested from its slots (nxt) and the slots of chunk c + 2 into cur.
+// one chunk (range m; slots cur, blocks val): every x the chunk needs is read
+// first, then the blocks of the next chunk (range mn) are requested from its
+// slots (nxt) and the slots of the chunk after (range ma) into cur.
 // No slot of a chunk reads an x that another slot of it writes (its columns
 // are rows of earlier levels, and a row has one segment per chunk), so the
 // entries' x_j and the rows' own x_i are all read before any is written: one
-// LDS round trip per chunk.  A chunk spans whole 64-slot windows, so a wave
-// whose window starts inside it has every lane on a slot of it: a slot
-// without an entry (column 0) reads the zero pair X[-2], X[-1] and forms a
-// zero product without a test; a lane without a row reads x_0 (a broadcast,
-// discarded).  The reads are unconditional, which keeps the wait for the
-// two ranges exact.  Returns mn.
-template <typename T, int SP, bool TR = false>
-__device__ __forceinline__ int4 slot_chunk(const int4 *slot, const int4 *swc,
-                                           const B4<T> *A, T *X, const int4 m,
-                                           bool bw, SlotIdx<SP> &cur,
-                                           const SlotVal<T, SP> &val,
-                                           int c_next, bool next_bw,
-                                           const SlotIdx<SP> &nxt,
-                                           SlotVal<T, SP> &nval, int c_after) {
+// LDS round trip per chunk.  A slot without an entry (column 0) reads the zero
+// pair X[-2], X[-1] and forms a zero product without a test; a lane without a
+// row reads x_0 (a broadcast, discarded).
+// What a wave does for a chunk it has no slot in is a few scalar tests: with
+// sixteen waves a chunk's time is what they issue, and most chunks of the
+// upper levels hold one to four waves' slots.
+template <typename T, int SP, bool TR>
+__device__ __forceinline__ void slot_chunk(const int4 *slot, const B4<T> *A, T *X, int wv,
+                                           int2 m, int2 mn, int2 ma, bool bw, bool next_bw,
+                                           SlotIdx<SP> &cur, const SlotVal<T, SP> &val,
+                                           const SlotIdx<SP> &nxt, SlotVal<T, SP> &nval) {
+  // in every wave: under a test the compiler would wait again at the use of
+  // the blocks, and so for the loads requested below
   __builtin_amdgcn_s_waitcnt(WAIT_VMCNT0);
-  int4 mn = swc[c_next], ma = swc[c_after];
   int lead[SP], lg[SP];
   T y0[SP], y1[SP], x0[SP], x1[SP];
 #pragma unroll
-  for (int k = 0; k < SP; k++) {
-    const int y = pinned(cur.s[k].y), z = pinned(cur.s[k].z);
-    const int cc = (y & ((1 << SLOT_LG_SHIFT) - 1)) - 1;
-    lead[k] = z;
-    lg[k] = y >> SLOT_LG_SHIFT;
-    const int ii = max(z, 0) & (SLOT_NOT_LAST - 1);
-    y0[k] = X[2 * cc];
-    y1[k] = X[2 * cc + 1];
-    x0[k] = X[2 * ii];
-    x1[k] = X[2 * ii + 1];
-  }
-  mn.x = __builtin_amdgcn_readfirstlane(mn.x);
-  mn.y = __builtin_amdgcn_readfirstlane(mn.y);
-  mn.z = __builtin_amdgcn_readfirstlane(mn.z);
-  ma.x = __builtin_amdgcn_readfirstlane(ma.x);
-  ma.y = __builtin_amdgcn_readfirstlane(ma.y);
-  nval = slot_values<T, SP, TR>(A, mn, next_bw, nxt);
-  cur = slot_index<SP>(slot, ma);
-  T p0[SP], p1[SP];
-#pragma unroll
-  for (int k = 0; k < SP; k++) {
-    const int q = m.x + (int)threadIdx.x + k * (int)blockDim.x;
-    if (wave_any(q, m.y)) {
-      const B4<T> &a = val.a[k];
-      if (TR) {   // the block (col, row) used transposed
-        p0[k] = a.a * y0[k] + a.c * y1[k];
-        p1[k] = a.b * y0[k] + a.d * y1[k];
-      } else {
-        p0[k] = a.a * y0[k] + a.b * y1[k];
-        p1[k] = a.c * y0[k] + a.d * y1[k];
-      }
+  for (int k = 0; k < SP; k++)
+    if (slot_on(m, wv, k)) {
+      const int y = pinned(cur.s[k].y), z = pinned(cur.s[k].z);
+      const int cc = (y & ((1 << SLOT_LG_SHIFT) - 1)) - 1;
+      lead[k] = z;
+      lg[k] = y >> SLOT_LG_SHIFT;
+      const int ii = max(z, 0) & (SLOT_NOT_LAST - 1);
+      y0[k] = X[2 * cc];
+      y1[k] = X[2 * cc + 1];
+      x0[k] = X[2 * ii];
+      x1[k] = X[2 * ii + 1];
     }
-  }
+  slot_values<T, SP, TR>(A, mn, wv, next_bw, nxt, nval);
+  slot_index<SP>(slot, ma, wv, cur);
 #pragma unroll
-  for (int k = 0; k < SP; k++) {
-    const int q = m.x + (int)threadIdx.x + k * (int)blockDim.x;
-    if (wave_any(q, m.y)) {
+  for (int k = 0; k < SP; k++)
+    if (slot_on(m, wv, k)) {
+      const B4<T> &a = val.a[k];
+      T p0, p1;
+      if (TR) {   // the block (col, row) used transposed
+        p0 = a.a * y0[k] + a.c * y1[k];
+        p1 = a.b * y0[k] + a.d * y1[k];
+      } else {
+        p0 = a.a * y0[k] + a.b * y1[k];
+        p1 = a.c * y0[k] + a.d * y1[k];
+      }
       // groups come largest first, each aligned to its size, so the wave's
       // first lane starts its largest group: the steps that group needs
-      slot_group_sum(p0[k], p1[k], lg[k], __builtin_amdgcn_readfirstlane(lg[k]));
+      slot_group_sum(p0, p1, lg[k], __builtin_amdgcn_readfirstlane(lg[k]));
       if (lead[k] >= 0) {
         // a row's earlier segments only subtract; its last one (or its only
         // one) also applies the pivot inverse in the backward sweep
         const int i = lead[k] & (SLOT_NOT_LAST - 1);
-        const T u0 = x0[k] - p0[k], u1 = x1[k] - p1[k];
+        const T u0 = x0[k] - p0, u1 = x1[k] - p1;
         if ((TR ? !bw : bw) && !(lead[k] & SLOT_NOT_LAST)) {
           const B4<T> &D = val.d[k];
           if (TR) {   // the pivot inverse transposed
@@ -2275,9 +2257,7 @@ __device__ __forceinline__ int4 slot_chunk(const int4 *slot, const int4 *swc,
         }
       }
     }
-  }
   __syncthreads();
-  return mn;
 }
 
 template <typename T, int SP, bool TR = false>
@@ -2295,27 +2275,40 @@ __device__ __forceinline__ void lu_sweeps_slot(const B4<T> *A, const B4<T> *Ti,
     if (tail) tail_rows<T>(A, Ti, X, rs, P, TR);
     return;
   }
-  const int cl = nc - 1;
+  const int lane = (int)threadIdx.x & 63;
+  const int wv = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  // the ranges of 64 chunks, one per lane, read with v_readlane (past the last
+  // chunk: empty)
+  int tx, ty;
+  auto load_ranges = [&](int c) {
+    const int4 v = swc[min(c + lane, nc - 1)];
+    tx = v.x;
+    ty = c + lane < nc ? v.y : v.x;
+  };
+  auto range = [&](int c) {
+    if (((c - c0) & 63) == 0) load_ranges(c);
+    int2 m;
+    m.x = __builtin_amdgcn_readlane(tx, (c - c0) & 63);
+    m.y = __builtin_amdgcn_readlane(ty, (c - c0) & 63);
+    return m;
+  };
   SlotIdx<SP> ia, ib;
   SlotVal<T, SP> va, vb;
-  int4 m = swc[c0];
-  m.x = __builtin_amdgcn_readfirstlane(m.x);
-  m.y = __builtin_amdgcn_readfirstlane(m.y);
-  m.z = __builtin_amdgcn_readfirstlane(m.z);
-  ia = slot_index<SP>(slots, m);
+  int2 m = range(c0), mn = range(c0 + 1);
+  slot_index<SP>(slots, m, wv, ia);
   __builtin_amdgcn_s_waitcnt(WAIT_VMCNT0);
-  va = slot_values<T, SP, TR>(A, m, c0 >= nfw, ia);
-  ib = slot_index<SP>(slots, swc[min(c0 + 1, cl)]);
+  slot_values<T, SP, TR>(A, m, wv, c0 >= nfw, ia, va);
+  slot_index<SP>(slots, mn, wv, ib);
   for (int c = c0; c < nc; c += 2) {
     if (c == nfw && tail) tail_rows<T>(A, Ti, X, rs, P, TR);
-    m = slot_chunk<T, SP, TR>(slots, swc, A, X, m, c >= nfw, ia, va,
-                              min(c + 1, cl), min(c + 1, cl) >= nfw, ib, vb,
-                              min(c + 2, cl));
+    int2 ma = range(c + 2);
+    slot_chunk<T, SP, TR>(slots, A, X, wv, m, mn, ma, c >= nfw, c + 1 >= nfw, ia, va, ib, vb);
     if (c + 1 >= nc) break;
     if (c + 1 == nfw && tail) tail_rows<T>(A, Ti, X, rs, P, TR);
-    m = slot_chunk<T, SP, TR>(slots, swc, A, X, m, c + 1 >= nfw, ib, vb,
-                              min(c + 2, cl), min(c + 2, cl) >= nfw, ia, va,
-                              min(c + 3, cl));
+    m = ma;
+    ma = range(c + 3);
+    slot_chunk<T, SP, TR>(slots, A, X, wv, mn, m, ma, c + 1 >= nfw, c + 2 >= nfw, ib, vb, ia, va);
+    mn = ma;
   }
   if (nc == nfw && tail) tail_rows<T>(A, Ti, X, rs, P, TR);
 }
@@ -2770,8 +2763,9 @@ __global__ void k_adj_solve(DevTopo g, DevInst d, const B4<double> *LU,
 // the adjoint solve J^T lambda = g in the slot form (X in LDS): the
 // transposed slots of the Newton sweeps, U^T forward with the pivots, the
 // tail by its transposed inverse, L^T backward; one workgroup per instance
+// (512 lanes take SP = 2 for chunks up to 1024 slots, 4 for longer ones)
 template <int SP>
-__global__ void __launch_bounds__(SLOT_CHUNK / SP)
+__global__ void __launch_bounds__(512)
 k_adj_solve_slot(DevTopo g, DevInst d, const B4<double> *LU, const B4<double> *TL,
                  const double *G, double *lam, SolvePlan P) {
   __shared__ double Xs[SOLVE_LDS_BYTES / sizeof(double)];
@@ -2950,6 +2944,7 @@ template __global__ void k_lu_solve<double, 1>(DevTopo, DevInst, const B4<double
 template __global__ void k_lu_solve<double, 2>(DevTopo, DevInst, const B4<double> *, const B4<double> *, int, int, SolvePlan, int, int, double *);
 template __global__ void k_lu_solve<double, 4>(DevTopo, DevInst, const B4<double> *, const B4<double> *, int, int, SolvePlan, int, int, double *);
 template __global__ void k_lu_solve<double, 8>(DevTopo, DevInst, const B4<double> *, const B4<double> *, int, int, SolvePlan, int, int, double *);
+template __global__ void k_adj_solve_slot<2>(DevTopo, DevInst, const B4<double> *, const B4<double> *, const double *, double *, SolvePlan);
 template __global__ void k_adj_solve_slot<4>(DevTopo, DevInst, const B4<double> *, const B4<double> *, const double *, double *, SolvePlan);
 
 }  // namespace bpf

@@ -423,7 +423,7 @@ bool analyse(int n, int m, const int *from, const int *to, const int *type,
   }
   S.prm.tail_limit = prm.tail_limit ? prm.tail_limit : TAIL_MAX;
   S.prm.chunk_pairs = prm.chunk_pairs ? prm.chunk_pairs : CHUNK_PAIRS;
-  S.prm.slot_chunk = prm.slot_chunk ? prm.slot_chunk : SLOT_CHUNK;
+  S.prm.slot_chunk = prm.slot_chunk ? prm.slot_chunk : SLOT_LANES;
   S.prm.ordering = prm.ordering;
   S.n = n;
   S.m = m;
@@ -1130,7 +1130,7 @@ bool analyse(int n, int m, const int *from, const int *to, const int *type,
   for (size_t c = 0; c < S.sw_cmax.size(); c++)
     if (S.sw_chunk[4 * c + 3] - S.sw_chunk[4 * c + 2] > SWEEP_CHUNK) S.sw_ok = 0;
   // slot form: rows of a level (longest first, so lane groups shrink and
-  // stay aligned) packed into chunks of at most SLOT_CHUNK slots.  A row of
+  // stay aligned) packed into chunks of at most prm.slot_chunk slots.  A row of
   // more than 64 entries is cut into segments of 64: segment j of every
   // such row goes into the chunks of pass j of the level (a new chunk starts
   // with each pass, so no chunk holds two segments of one row); each
@@ -1204,12 +1204,20 @@ bool analyse(int n, int m, const int *from, const int *to, const int *type,
     }
     return nch;
   };
-  S.sl_nfw = slots(S.fw_ptr, S.fw_rows, S.nfw, true, false, S.sl_chunk, S.sl_slot);
-  S.sl_nbw = slots(S.bw_ptr, S.bw_rows, S.nbw, false, false, S.sl_chunk, S.sl_slot);
-  S.sl_ok = S.sl_nfw + S.sl_nbw <= MAX_CHUNKS;
-  S.sl_nfw_t = slots(S.fw_ptr, S.fw_rows, S.nfw, true, true, S.sl_chunk_t, S.sl_slot_t);
-  S.sl_nbw_t = slots(S.bw_ptr, S.bw_rows, S.nbw, false, true, S.sl_chunk_t, S.sl_slot_t);
-  S.sl_ok_t = S.sl_nfw_t + S.sl_nbw_t <= MAX_CHUNKS;
+  auto slot_plan = [&] {
+    for (std::vector<int> *v : {&S.sl_chunk, &S.sl_slot, &S.sl_chunk_t, &S.sl_slot_t}) v->clear();
+    S.sl_nfw = slots(S.fw_ptr, S.fw_rows, S.nfw, true, false, S.sl_chunk, S.sl_slot);
+    S.sl_nbw = slots(S.bw_ptr, S.bw_rows, S.nbw, false, false, S.sl_chunk, S.sl_slot);
+    S.sl_ok = S.sl_nfw + S.sl_nbw <= MAX_CHUNKS;
+    S.sl_nfw_t = slots(S.fw_ptr, S.fw_rows, S.nfw, true, true, S.sl_chunk_t, S.sl_slot_t);
+    S.sl_nbw_t = slots(S.bw_ptr, S.bw_rows, S.nbw, false, true, S.sl_chunk_t, S.sl_slot_t);
+    S.sl_ok_t = S.sl_nfw_t + S.sl_nbw_t <= MAX_CHUNKS;
+  };
+  slot_plan();
+  if (!prm.slot_chunk && !(S.sl_ok && S.sl_ok_t)) {
+    S.prm.slot_chunk = SLOT_CHUNK;
+    slot_plan();
+  }
   return true;
 }
 

@@ -19,6 +19,14 @@ constexpr int TASK_POS_MASK = (1 << 28) - 1;
 constexpr int CHUNK_PAIRS = 4096;    // products per factorization chunk (LDS)
 constexpr int SWEEP_CHUNK = 2048;    // entries per sweep chunk (LDS)
 constexpr int SLOT_CHUNK = 2048;     // lane slots per sweep chunk, slot form
+// the chunk length taken by default: one slot per lane of the default sweep
+// workgroup.  Two per lane halve the chunks of the widest levels but double
+// the registers (64 spilled in FP64 at 1024 lanes), and a chunk costs what
+// its waves issue, not its barrier.  A sweep pass, 2048 / 1024 / 512 slots:
+// 9241 buses, 1 instance, FP32 77 / 69 / 84 us, FP64 117 / 69 / 76; 200
+// instances 109 / 105 / -, 184 / 123 / -; 1354 buses x 1000 107 / 98 / -,
+// 152 / 104 / -
+constexpr int SLOT_LANES = 1024;
 constexpr int SLOT_LG_SHIFT = 27;    // slot column word: column + 1 | log2 group << 27
 constexpr int SLOT_NOT_LAST = 1 << 30;  // slot row word: a segment before the row's last
 constexpr int MAX_CHUNKS = 512;      // chunk tables the kernels keep in LDS
@@ -29,9 +37,10 @@ constexpr int SPLIT_VARIANTS = 3;    // splits into 2, 4 and 8 workgroups
 // (with the chunk tables, which the tail no longer needs, in the same space)
 constexpr int TAIL_STAGE_MAX = 5760;
 
-// tile sizes of the schedules (0 = the largest the kernels hold): pivots
-// of the dense tail, products per factorization chunk, lane slots per
-// slot-form sweep chunk
+// tile sizes of the schedules: pivots of the dense tail, products per
+// factorization chunk (0 = the largest the kernels hold), lane slots per
+// slot-form sweep chunk (0 = SLOT_LANES; SLOT_CHUNK where the chunks would
+// then not fit the kernels' table)
 struct AnalysisParams {
   int tail_limit = 0, chunk_pairs = 0, slot_chunk = 0;
   // bus ordering: 0 minimum degree, 1 minimum degree reordered to the least
@@ -43,7 +52,7 @@ struct AnalysisParams {
 };
 
 struct Symbolic {
-  AnalysisParams prm;   // the values used (0s replaced by the maxima)
+  AnalysisParams prm;   // the values used (0s replaced by the defaults)
   int n = 0, m = 0, nb = 0;
   // Ybus pattern over all buses (every branch, in service or not: outages
   // only zero values, as the reference keeps the structure, makeYbus.h:69-71)

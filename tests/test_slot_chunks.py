@@ -1,0 +1,60 @@
+"""Lane slots per chunk of the slot-form sweeps: chunks of one slot per lane by
+default, of two where the chunk table would not hold the others (host only);
+on the GPU the adjoint's sweeps agree with the level rows at every chunk
+length.  Tolerance: another summation order of the same J^T lambda = g, as in
+the adjoint's own test of its two forms (1e-9 of the largest entry)."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+from mapol_amd import engine, synth
+
+
+def _tree(n, seed=2):
+    """a radial grid: bus i hangs on a random earlier one"""
+    rng = np.random.default_rng(seed)
+    case = synth.workload("pf118x200", T=1)[0]
+    f = {k: np.zeros(n, v.dtype) for k, v in case.__dict__.items()
+         if isinstance(v, np.ndarray) and v.shape == case.Pd.shape}
+    f["bus_type"] = np.ones(n, case.bus_type.dtype)
+    f["bus_type"][0] = 3
+    f["Vm"] = np.ones(n)
+    for k in ("R", "X", "B", "tap", "shift"):
+        f[k] = np.full(n - 1, 0.1 if k == "X" else 0.0)
+    f["br_status"] = np.ones(n - 1, case.br_status.dtype)
+    f["br_to"] = np.arange(1, n, dtype=case.br_to.dtype)
+    f["br_from"] = (rng.random(n - 1) * np.arange(1, n)).astype(case.br_from.dtype)
+    for k in ("gen_bus", "Pg", "Qg", "Qmax", "Qmin", "VG", "gen_status"):
+        f[k] = getattr(case, k)[:1].copy()
+    f["gen_bus"][0] = 0
+    return synth.Case(**{**case.__dict__, **f, "xy": None})
+
+
+@pytest.mark.parametrize("n,limit", [(20000, 1024), (330000, 2048)])
+def test_default_chunk_length(n, limit):
+    keep, info = [], engine.BpfInfo()
+    s = engine._case_struct(_tree(n), keep)
+    assert engine.load_library().bpf_analyse(C.byref(s), C.byref(info), *([None] * 21)) == 0
+    chunks = info.slot_fw_chunks + info.slot_bw_chunks
+    assert 0 < chunks <= 512
+    # every slot of a chunk of at most `limit`: the bound from both sides
+    assert info.slots <= chunks * limit
+    if limit == 2048:
+        assert info.slots > 512 * 1024
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("slot_chunk", [0, 64, 1024, 1088, 2048])
+def test_adjoint_at_every_chunk_length(slot_chunk):
+    case, cont = synth.workload("pf1354x200", T=3)
+    e = engine.Engine(case, tol=1e-12, maxit_nr=20, slot_chunk=slot_chunk)
+    e.set_instances(br_on=cont.br_on, gen_on=cont.gen_on)
+    e.solve()
+    rate = np.linspace(0.5, 2.0, case.nbranch)
+    got = e.adjoint(rate=rate, w=1.0)
+    e.set_schedule(sweep_form=3)
+    ref = e.adjoint(rate=rate, w=1.0)
+    e.close()
+    for k in ("grad_P", "grad_Q", "grad_x"):
+        assert np.abs(got[k] - ref[k]).max() <= 1e-9 * np.abs(ref[k]).max(), k
