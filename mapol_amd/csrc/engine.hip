@@ -12,6 +12,7 @@
 #include <mutex>
 #include <numeric>
 #include <string>
+#include <thread>
 #include <type_traits>
 #include <utility>
 #include <vector>
@@ -62,6 +63,11 @@ static int sweep_mode(const Symbolic &S, size_t scalar, int use_lds, int form,
 static dim3 xgrid(int T, size_t count, unsigned threads) {
   return dim3(8u * div_up((size_t)T, 8) * div_up(count, threads));
 }
+
+// results leave through pinned memory: OUT_PARTS copying threads with two
+// buffers of OUT_CHUNK bytes each
+constexpr size_t OUT_CHUNK = 1 << 20;
+constexpr int OUT_PARTS = 4;
 
 struct bpf_engine {
   bpf_options opt;
@@ -119,11 +125,13 @@ struct bpf_engine {
   void *d_UPD = nullptr;
   struct AdjBufs {
     double *rate = nullptr, *G = nullptr, *lam = nullptr, *gP = nullptr,
-           *gQ = nullptr, *gx = nullptr, *obj = nullptr;
+           *gQ = nullptr, *gx = nullptr, *obj = nullptr, *st = nullptr;
   } adj;
   cd *d_Sf = nullptr, *d_St = nullptr;
   double *d_loss = nullptr;
   int *h_count = nullptr;       // pinned
+  char *h_out = nullptr;        // pinned, results on their way out (to_host)
+  hipEvent_t h_ev[2 * OUT_PARTS] = {};
   // launch shapes
   int lu_threads = 1024, solve_threads = 1024, mis_threads = 256;
   int max_lds = 65536;
@@ -277,6 +285,9 @@ extern "C" void bpf_destroy(bpf_engine *e) {
   free_pool(e->owned);
   if (e->d_bus_stage) hipFree(e->d_bus_stage);
   if (e->h_count) hipHostFree(e->h_count);
+  if (e->h_out) hipHostFree(e->h_out);
+  for (hipEvent_t ev : e->h_ev)
+    if (ev) hipEventDestroy(ev);
   if (e->stream) hipStreamDestroy(e->stream);
   delete e;
 }
@@ -299,23 +310,100 @@ static bpf_status bus_stage(bpf_engine *e, size_t bytes) {
   return BPF_OK;
 }
 
-template <class V>
-static bpf_status bus_rows_download(bpf_engine *e, const void *dsrc, V *dst, size_t T) {
-  const size_t cnt = T * e->n, bytes = sizeof(V) * cnt;
-  if (cnt == 0) return BPF_OK;
-  if (!e->opt.bus_numbering) {
-    HIPCHK(hipMemcpyAsync(dst, dsrc, bytes, hipMemcpyDeviceToHost, e->stream));
-    HIPCHK(hipStreamSynchronize(e->stream));
+// device memory to the caller's, after the work queued on the engine's stream:
+// through pinned buffers, the copy of one chunk running while the host stores
+// the one before (into pageable memory the runtime does both in turn: 18 GB/s
+// where the link gives 57).  Copies of OUT_SPLIT bytes and more are shared by
+// OUT_PARTS threads: storing into a fresh array is bound by its page faults
+// (32 MB of voltages: one thread 2.6 ms, four 1.1, the runtime's copy 3.4).
+// store(offset, data, bytes) takes a chunk; offsets are multiples of OUT_CHUNK.
+constexpr size_t OUT_SPLIT = 8u << 20;
+
+template <class Store>
+static bpf_status to_host(bpf_engine *e, const void *dsrc, size_t bytes, const Store &store) {
+  const size_t nc = (bytes + OUT_CHUNK - 1) / OUT_CHUNK;
+  const int parts = bytes >= OUT_SPLIT ? OUT_PARTS : 1;
+  if (!e->h_out) {
+    std::vector<char> buf(std::min(bytes, OUT_CHUNK));
+    for (size_t c = 0; c < nc; c++) {
+      const size_t b = std::min(OUT_CHUNK, bytes - c * OUT_CHUNK);
+      HIPCHK(hipMemcpyAsync(buf.data(), (const char *)dsrc + c * OUT_CHUNK, b,
+                            hipMemcpyDeviceToHost, e->stream));
+      HIPCHK(hipStreamSynchronize(e->stream));
+      store(c * OUT_CHUNK, buf.data(), b);
+    }
     return BPF_OK;
   }
-  bpf_status s = bus_stage(e, bytes);
+  int dev = 0;
+  HIPCHK(hipGetDevice(&dev));
+  hipError_t res[OUT_PARTS] = {};
+  auto part = [&](int p) {
+    const size_t c0 = nc * p / parts, c1 = nc * (p + 1) / parts;
+    hipError_t r = p ? hipSetDevice(dev) : hipSuccess;
+    size_t asked = c0;
+    for (size_t c = c0; c < c1 && r == hipSuccess; c++) {
+      for (; asked < std::min(c + 2, c1) && r == hipSuccess; asked++) {
+        const int k = 2 * p + (int)(asked & 1);
+        r = hipMemcpyAsync(e->h_out + k * OUT_CHUNK, (const char *)dsrc + asked * OUT_CHUNK,
+                           std::min(OUT_CHUNK, bytes - asked * OUT_CHUNK),
+                           hipMemcpyDeviceToHost, e->stream);
+        if (r == hipSuccess) r = hipEventRecord(e->h_ev[k], e->stream);
+      }
+      const int k = 2 * p + (int)(c & 1);
+      if (r == hipSuccess) r = hipEventSynchronize(e->h_ev[k]);
+      if (r == hipSuccess)
+        store(c * OUT_CHUNK, e->h_out + k * OUT_CHUNK, std::min(OUT_CHUNK, bytes - c * OUT_CHUNK));
+    }
+    res[p] = r;
+  };
+  std::thread th[OUT_PARTS];
+  for (int p = 1; p < parts; p++) {
+    try {
+      th[p] = std::thread(part, p);
+    } catch (const std::exception &) {
+      part(p);                    // no thread to be had: here, in turn
+    }
+  }
+  part(0);
+  for (std::thread &t : th)
+    if (t.joinable()) t.join();
+  for (hipError_t r : res)
+    if (r != hipSuccess) {
+      hipStreamSynchronize(e->stream);   // no copy into the buffers outlives the call
+      e->err = std::string("copy to the host: ") + hipGetErrorString(r);
+      return BPF_ERR_HIP;
+    }
+  return BPF_OK;
+}
+
+template <class V>
+static bpf_status to_host(bpf_engine *e, const void *dsrc, V *dst, size_t cnt) {
+  return to_host(e, dsrc, sizeof(V) * cnt, [&](size_t off, const char *p, size_t b) {
+    memcpy((char *)dst + off, p, b);
+  });
+}
+
+// T rows of per-bus values of the device, in the caller's numbering: where
+// they lie (the staging buffer, or dsrc itself)
+template <class V>
+static bpf_status bus_rows_gather(bpf_engine *e, const void *dsrc, size_t T, const void **out) {
+  *out = dsrc;
+  const size_t cnt = T * e->n;
+  if (!e->opt.bus_numbering || cnt == 0) return BPF_OK;
+  bpf_status s = bus_stage(e, sizeof(V) * cnt);
   if (s) return s;
   hipLaunchKernelGGL(k_bus_gather<V>, dim3(div_up(cnt, 256)), dim3(256), 0, e->stream,
                      (const V *)dsrc, (V *)e->d_bus_stage, e->d_bus_int, e->n, (int)T);
   HIPCHK(hipGetLastError());
-  HIPCHK(hipMemcpyAsync(dst, e->d_bus_stage, bytes, hipMemcpyDeviceToHost, e->stream));
-  HIPCHK(hipStreamSynchronize(e->stream));
+  *out = e->d_bus_stage;
   return BPF_OK;
+}
+
+template <class V>
+static bpf_status bus_rows_download(bpf_engine *e, const void *dsrc, V *dst, size_t T) {
+  const void *src;
+  bpf_status s = bus_rows_gather<V>(e, dsrc, T, &src);
+  return s ? s : to_host(e, src, dst, T * e->n);
 }
 
 // the caller's T rows of voltages into the engine's V (queued on the
@@ -501,6 +589,12 @@ extern "C" bpf_status bpf_create(const bpf_case *c, const bpf_options *o,
                                hipDeviceAttributeMaxSharedMemoryPerBlock, e->dev));
   HIPCHK(hipDeviceGetAttribute(&e->num_cu, hipDeviceAttributeMultiprocessorCount,
                                e->dev));
+  if (hipHostMalloc((void **)&e->h_out, 2 * OUT_PARTS * OUT_CHUNK, hipHostMallocDefault) !=
+      hipSuccess) {
+    (void)hipGetLastError();
+    e->h_out = nullptr;           // to_host then copies without it
+  }
+  for (hipEvent_t &ev : e->h_ev) HIPCHK(hipEventCreateWithFlags(&ev, hipEventDisableTiming));
   HIPCHK(hipHostMalloc((void **)&e->h_count, sizeof(int) * bpf_engine::MAX_SPLIT,
                        hipHostMallocDefault));
   const Symbolic &S = e->S;
@@ -1489,22 +1583,47 @@ extern "C" bpf_status bpf_get_results(bpf_engine *e, double *V, int32_t *its,
                                       int32_t *bus_type) {
   if (!e) return BPF_ERR_INVALID_ARG;
   if (!e->solved) { e->err = "no solution yet"; return BPF_ERR_STATE; }
-  const size_t T = e->T, n = e->n;
+  const size_t T = e->T, n = e->n, cnt = T * n;
   bpf_status s;
+  auto states = [&](const InstState *st) {
+    for (size_t t = 0; t < T; t++) {
+      if (its) its[t] = st[t].it_total;
+      if (verdict) verdict[t] = st[t].verdict;
+      if (norm) norm[t] = st[t].norm;
+      if (rounds) rounds[t] = st[t].rounds;
+    }
+  };
+  const size_t o_st = sizeof(cd) * cnt, o_ls = o_st + sizeof(InstState) * T,
+               o_ty = o_ls + sizeof(double) * T;
+  if (e->h_out && o_ty + cnt <= 2 * OUT_CHUNK) {
+    // small batches: one kernel gathers everything into the pinned buffer,
+    // one wait (four copies and a wait each took 85 us for 14 buses)
+    InstState *st = (InstState *)(e->h_out + o_st);
+    double *ls = (double *)(e->h_out + o_ls);
+    const int8_t *ty = (const int8_t *)(e->h_out + o_ty);
+    hipLaunchKernelGGL(k_results, dim3(div_up(std::max(cnt, T), 256)), dim3(256), 0, e->stream,
+                       e->d, e->d_loss, e->opt.bus_numbering ? e->d_bus_int : nullptr, (int)n,
+                       (cd *)e->h_out, st, ls, (int8_t *)ty);
+    HIPCHK(hipGetLastError());
+    HIPCHK(hipStreamSynchronize(e->stream));
+    if (V) memcpy(V, e->h_out, o_st);
+    states(st);
+    if (loss) memcpy(loss, ls, sizeof(double) * T);
+    if (bus_type)
+      for (size_t k = 0; k < cnt; k++) bus_type[k] = ty[k];
+    return BPF_OK;
+  }
   if (V && (s = bus_rows_download(e, e->d.V, (cd *)V, T))) return s;
   std::vector<InstState> st(T);
-  HIPCHK(hipMemcpy(st.data(), e->d.st, sizeof(InstState) * T, hipMemcpyDeviceToHost));
-  for (size_t t = 0; t < T; t++) {
-    if (its) its[t] = st[t].it_total;
-    if (verdict) verdict[t] = st[t].verdict;
-    if (norm) norm[t] = st[t].norm;
-    if (rounds) rounds[t] = st[t].rounds;
-  }
-  if (loss) HIPCHK(hipMemcpy(loss, e->d_loss, sizeof(double) * T, hipMemcpyDeviceToHost));
+  if ((s = to_host(e, e->d.st, st.data(), T))) return s;
+  states(st.data());
+  if (loss && (s = to_host(e, e->d_loss, loss, T))) return s;
   if (bus_type) {
-    std::vector<int8_t> ty(T * n);
-    if ((s = bus_rows_download(e, e->d.type, ty.data(), T))) return s;
-    for (size_t k = 0; k < T * n; k++) bus_type[k] = ty[k];
+    const void *src;
+    if ((s = bus_rows_gather<int8_t>(e, e->d.type, T, &src))) return s;
+    return to_host(e, src, cnt, [&](size_t off, const char *p, size_t b) {
+      for (size_t k = 0; k < b; k++) bus_type[off + k] = ((const int8_t *)p)[k];
+    });
   }
   return BPF_OK;
 }
@@ -1512,9 +1631,10 @@ extern "C" bpf_status bpf_get_results(bpf_engine *e, double *V, int32_t *its,
 extern "C" bpf_status bpf_get_branch_flows(bpf_engine *e, double *Sf, double *St) {
   if (!e) return BPF_ERR_INVALID_ARG;
   if (!e->solved) { e->err = "no solution yet"; return BPF_ERR_STATE; }
-  size_t bytes = sizeof(cd) * (size_t)e->T * e->m;
-  if (Sf) HIPCHK(hipMemcpy(Sf, e->d_Sf, bytes, hipMemcpyDeviceToHost));
-  if (St) HIPCHK(hipMemcpy(St, e->d_St, bytes, hipMemcpyDeviceToHost));
+  const size_t cnt = (size_t)e->T * e->m;
+  bpf_status s;
+  if (Sf && (s = to_host(e, e->d_Sf, (cd *)Sf, cnt))) return s;
+  if (St && (s = to_host(e, e->d_St, (cd *)St, cnt))) return s;
   return BPF_OK;
 }
 
@@ -1529,35 +1649,23 @@ extern "C" bpf_status bpf_get_branch_loading(bpf_engine *e, const double *rate,
       e->err = "branch ratings must be >= 0 (0: no rating)";
       return BPF_ERR_INVALID_ARG;
     }
-  std::vector<DBuf> tmp;
-  struct Free { std::vector<DBuf> &v; ~Free() { free_pool(v); } } fr{tmp};
-  void *p;
-  bpf_status s;
-  double *d_rate, *d_load = nullptr, *d_max;
-  int *d_over;
-  if ((s = dalloc(e, tmp, sizeof(double) * (size_t)std::max(m, 1), &p))) return s;
-  d_rate = (double *)p;
-  if (loading) {
-    if ((s = dalloc(e, tmp, sizeof(double) * (size_t)T * std::max(m, 1), &p))) return s;
-    d_load = (double *)p;
-  }
-  if ((s = dalloc(e, tmp, sizeof(int) * (size_t)T, &p))) return s;
-  d_over = (int *)p;
-  if ((s = dalloc(e, tmp, sizeof(double) * (size_t)T, &p))) return s;
-  d_max = (double *)p;
-  if (m) HIPCHK(hipMemcpy(d_rate, rate, sizeof(double) * m, hipMemcpyHostToDevice));
+  // ratings, counts, largest loadings and rows in the staging buffer, which
+  // the engine keeps (four allocations and their release took 200 us)
+  const size_t o_max = sizeof(double) * std::max(m, 1), o_over = o_max + sizeof(double) * T,
+               o_load = (o_over + sizeof(int) * T + 255) / 256 * 256;
+  bpf_status s = bus_stage(e, o_load + (loading ? sizeof(double) * (size_t)T * std::max(m, 1) : 0));
+  if (s) return s;
+  char *stage = (char *)e->d_bus_stage;
+  if (m) HIPCHK(hipMemcpyAsync(stage, rate, sizeof(double) * m, hipMemcpyHostToDevice, e->stream));
   hipLaunchKernelGGL(k_branch_report, dim3(T), dim3(256), 0, e->stream, e->g, T,
-                     e->d_Sf, e->d_St, d_rate, d_load, d_over, d_max);
+                     e->d_Sf, e->d_St, (const double *)stage,
+                     loading ? (double *)(stage + o_load) : nullptr,
+                     (int *)(stage + o_over), (double *)(stage + o_max));
   HIPCHK(hipGetLastError());
+  if (loading && (s = to_host(e, stage + o_load, loading, (size_t)T * m))) return s;
+  if (overloads && (s = to_host(e, stage + o_over, overloads, (size_t)T))) return s;
+  if (max_loading && (s = to_host(e, stage + o_max, max_loading, (size_t)T))) return s;
   HIPCHK(hipStreamSynchronize(e->stream));
-  if (loading)
-    HIPCHK(hipMemcpy(loading, d_load, sizeof(double) * (size_t)T * m,
-                     hipMemcpyDeviceToHost));
-  std::vector<int> ov(T);
-  HIPCHK(hipMemcpy(ov.data(), d_over, sizeof(int) * T, hipMemcpyDeviceToHost));
-  if (overloads) for (int t = 0; t < T; t++) overloads[t] = ov[t];
-  if (max_loading)
-    HIPCHK(hipMemcpy(max_loading, d_max, sizeof(double) * T, hipMemcpyDeviceToHost));
   return BPF_OK;
 }
 
@@ -2022,10 +2130,10 @@ extern "C" bpf_status bpf_adjoint(bpf_engine *e, const double *rate, double w,
   auto &a = e->adj;
   if (!a.G) {
     void *p;
-    double **dst[] = {&a.rate, &a.G, &a.lam, &a.gP, &a.gQ, &a.gx, &a.obj};
+    double **dst[] = {&a.rate, &a.G, &a.lam, &a.gP, &a.gQ, &a.gx, &a.obj, &a.st};
     const size_t cnt[] = {std::max<size_t>(m, 1), T * nb2, T * nb2, T * n, T * n,
-                          T * std::max<size_t>(m, 1), T};
-    for (int k = 0; k < 7; k++) {
+                          T * std::max<size_t>(m, 1), T, T * sizeof(InstState) / sizeof(double)};
+    for (int k = 0; k < 8; k++) {
       if ((s = dalloc(e, e->inst_owned, sizeof(double) * cnt[k], &p))) {
         a = bpf_engine::AdjBufs();
         return s;
@@ -2038,12 +2146,9 @@ extern "C" bpf_status bpf_adjoint(bpf_engine *e, const double *rate, double w,
                           e->stream));
   const double *d_rate = rate ? a.rate : nullptr;
   // only converged instances take part
-  std::vector<InstState> st(T), st2;
-  HIPCHK(hipMemcpy(st.data(), e->d.st, sizeof(InstState) * T, hipMemcpyDeviceToHost));
-  st2 = st;
-  for (auto &x : st2) x.done = x.verdict == BPF_V_CONVERGED ? 0 : 1;
-  HIPCHK(hipMemcpy(e->d.st, st2.data(), sizeof(InstState) * T, hipMemcpyHostToDevice));
   const unsigned TT = (unsigned)T;
+  hipLaunchKernelGGL(k_adj_states, dim3(div_up(T, 256)), dim3(256), 0, e->stream, e->d,
+                     (InstState *)a.st, 0);
   tbegin(e, "adjoint");
   hipLaunchKernelGGL(k_jacobian<double>, xgrid(TT, ((size_t)e->g.nJb + 1) / 2, 256),
                      dim3(256), 0, e->stream, e->g, e->d, LU, 0, -1);
@@ -2074,20 +2179,21 @@ extern "C" bpf_status bpf_adjoint(bpf_engine *e, const double *rate, double w,
   hipLaunchKernelGGL(k_objective, dim3(TT), dim3(256), 0, e->stream, e->g,
                      e->d, d_rate, w, a.obj);
   tend(e);
+  // factorization singularities are not expected at a converged point; keep
+  // the verdicts of the solve either way
+  hipLaunchKernelGGL(k_adj_states, dim3(div_up(T, 256)), dim3(256), 0, e->stream, e->d,
+                     (InstState *)a.st, 1);
   hipError_t r1 = hipStreamSynchronize(e->stream);
   hipError_t r2 = hipGetLastError();
   tcollect(e);
-  // factorization singularities are not expected at a converged point; keep
-  // the verdicts of the solve either way
-  HIPCHK(hipMemcpy(e->d.st, st.data(), sizeof(InstState) * T, hipMemcpyHostToDevice));
   if (r1 != hipSuccess || r2 != hipSuccess) {
     e->err = std::string("adjoint: ") + hipGetErrorString(r1 != hipSuccess ? r1 : r2);
     return BPF_ERR_HIP;
   }
   if (gP && (s = bus_rows_download(e, a.gP, gP, T))) return s;
   if (gQ && (s = bus_rows_download(e, a.gQ, gQ, T))) return s;
-  if (gx) HIPCHK(hipMemcpy(gx, a.gx, sizeof(double) * T * m, hipMemcpyDeviceToHost));
-  if (obj) HIPCHK(hipMemcpy(obj, a.obj, sizeof(double) * T, hipMemcpyDeviceToHost));
+  if (gx && (s = to_host(e, a.gx, gx, T * m))) return s;
+  if (obj && (s = to_host(e, a.obj, obj, T))) return s;
   return BPF_OK;
 }
 

@@ -2924,6 +2924,37 @@ __global__ void k_bus_gather(const V *src, V *dst, const int *map, int n, int T)
   dst[q] = src[t * (size_t)n + map[k]];
 }
 
+// the adjoint's instances: the states saved and every instance but the
+// converged ones left out (back = 0), or the saved ones put back
+__global__ void k_adj_states(DevInst d, InstState *saved, int back) {
+  const int t = blockIdx.x * blockDim.x + threadIdx.x;
+  if (t >= d.T) return;
+  if (back) {
+    d.st[t] = saved[t];
+  } else {
+    const InstState s = d.st[t];
+    saved[t] = s;
+    d.st[t].done = s.verdict == BPF_V_CONVERGED ? 0 : 1;
+  }
+}
+
+// a small batch's voltages, states, losses and bus types into one buffer
+// (map: the caller's bus numbering, or null)
+__global__ void k_results(DevInst d, const double *loss, const int *map, int n, cd *V,
+                          InstState *st, double *ls, int8_t *type) {
+  const size_t q = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (q < (size_t)n * d.T) {
+    const size_t t = q / (size_t)n, k = q - t * (size_t)n;
+    const size_t p = map ? t * (size_t)n + map[k] : q;
+    V[q] = d.V[p];
+    type[q] = d.type[p];
+  }
+  if (q < (size_t)d.T) {
+    st[q] = d.st[q];
+    ls[q] = loss[q];
+  }
+}
+
 // explicit instantiations used by the engine
 template __global__ void k_bus_gather<cd>(const cd *, cd *, const int *, int, int);
 template __global__ void k_bus_gather<double>(const double *, double *, const int *, int, int);

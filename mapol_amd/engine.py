@@ -417,18 +417,23 @@ class Engine:
 
     def results(self):
         T, n = self.T, self.case.nbus
-        V = np.zeros((T, n, 2))
-        its = np.zeros(T, np.int32)
-        ver = np.zeros(T, np.int32)
-        nrm = np.zeros(T)
-        loss = np.zeros(T)
-        rnd = np.zeros(T, np.int32)
-        bt = np.zeros((T, n), np.int32)
+        V = np.empty((T, n), np.complex128)
+        its = np.empty(T, np.int32)
+        ver = np.empty(T, np.int32)
+        nrm = np.empty(T)
+        loss = np.empty(T)
+        rnd = np.empty(T, np.int32)
+        bt = np.empty((T, n), np.int32)
         self._check(self.L.bpf_get_results(
-            self.h, _ptr(V, _pd), _ptr(its, _pi), _ptr(ver, _pi),
+            self.h, _ptr(V.view(np.float64), _pd), _ptr(its, _pi), _ptr(ver, _pi),
             _ptr(nrm, _pd), _ptr(loss, _pd), _ptr(rnd, _pi), _ptr(bt, _pi)),
             "bpf_get_results")
-        return dict(V=V[..., 0] + 1j * V[..., 1], iterations=its, verdict=ver,
+        # an instance that ended without a finite solution: infinite parts
+        # spread as in the product with 1j
+        for t in np.flatnonzero(ver != CONVERGED):
+            if not np.isfinite(V[t]).all():
+                V[t] = V[t].real + 1j * V[t].imag
+        return dict(V=V, iterations=its, verdict=ver,
                     norm=nrm, loss=loss, qlim_rounds=rnd, bus_type=bt)
 
     def branch_flows(self):
@@ -448,9 +453,9 @@ class Engine:
         rt = np.ascontiguousarray(rate, np.float64)
         if rt.shape != (m,):
             raise EngineError(f"rate must have shape ({m},)")
-        load = np.zeros((T, m))
-        over = np.zeros(T, np.int32)
-        mx = np.zeros(T)
+        load = np.empty((T, m))
+        over = np.empty(T, np.int32)
+        mx = np.empty(T)
         self._check(self.L.bpf_get_branch_loading(self.h, _ptr(rt, _pd),
                                                   _ptr(load, _pd), _ptr(over, _pi),
                                                   _ptr(mx, _pd)),
@@ -574,10 +579,10 @@ class Engine:
 
     def adjoint(self, rate=None, w=0.0):
         T, n, m = self.T, self.case.nbus, self.case.nbranch
-        gP = np.zeros((T, n))
-        gQ = np.zeros((T, n))
-        gx = np.zeros((T, m))
-        obj = np.zeros(T)
+        gP = np.empty((T, n))
+        gQ = np.empty((T, n))
+        gx = np.empty((T, m))
+        obj = np.empty(T)
         r = None if rate is None else np.ascontiguousarray(rate, np.float64)
         self._check(self.L.bpf_adjoint(self.h, _ptr(r, _pd), float(w),
                                        _ptr(gP, _pd), _ptr(gQ, _pd),
