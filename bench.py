@@ -55,7 +55,8 @@ def algorithmic_bytes(info, case, T, its_total, s, refine):
     first = (4 * s * (nLU - nL) + 4 * s * nb + 16 * nb) if fused \
         else (4 * s * nLU + 32 * nb)
     per_inst = {
-        "ybus": 16 * nY + 9 * m + 8 * n,
+        "init": 16 * nY + 50 * n,
+        "ybus": 9 * m,
         "mismatch": 16 * nY + 48 * n + 16 * nb + n,
         "jacobian": 16 * nY + 32 * n + n + 4 * s * nJ,
         "lu_factor": 4 * s * nJ + 4 * s * nLU,
@@ -67,7 +68,7 @@ def algorithmic_bytes(info, case, T, its_total, s, refine):
         "loss": 16 * n + 41 * m,
     }
     launches_inst = {
-        "ybus": T, "loss": T, "mismatch": T + its_total,
+        "init": T, "ybus": T, "loss": T, "mismatch": T + its_total,
         "jacobian": its_total, "lu_factor": its_total, "lu_solve": its_total,
         "residual": its_total,
         "update": its_total,

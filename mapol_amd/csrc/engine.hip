@@ -650,6 +650,33 @@ extern "C" bpf_status bpf_create(const bpf_case *c, const bpf_options *o,
     g.ys = (const cd *)p1;
     g.ejs = (const cd *)p2;
   }
+  {
+    // the entries at the case's own taps (another tap computes its entry)
+    const size_t cnt = 4 * (size_t)std::max(e->m, 1);
+    void *p1, *p2 = nullptr;
+    std::vector<int> at(4 * (size_t)std::max(e->m, 1));
+    for (const auto &l : {std::make_pair(&S.yf_ptr, &S.yf_item), std::make_pair(&S.yt_ptr, &S.yt_item)})
+      for (int p = 0; p < g.nnzY; p++)
+        for (int q = (*l.first)[p]; q < (*l.first)[p + 1]; q++) at[(*l.second)[q]] = p;
+    const std::vector<uint8_t> on0(e->br_status);
+    UP(g.tap0, nonemptyd(e->tap)); UP(g.on0, nonempty8(on0)); UP(g.ybr, at);
+    void *p3;
+    if ((s = dalloc(e, e->owned, sizeof(cd) * cnt, &p1))) return s;
+    if (e->opt.alg != BPF_NR && (s = dalloc(e, e->owned, sizeof(double2) * cnt, &p2))) return s;
+    if ((s = dalloc(e, e->owned, sizeof(cd) * (size_t)g.nnzY, &p3))) return s;
+    if (e->m) {
+      hipLaunchKernelGGL(k_branch_entries, dim3(div_up(cnt, 256)), dim3(256), 0, e->stream, g,
+                         (int)e->opt.alg, (cd *)p1, (double2 *)p2);
+      HIPCHK(hipGetLastError());
+    }
+    hipLaunchKernelGGL(k_ybus_base, dim3(div_up(g.nnzY, 256)), dim3(256), 0, e->stream, g,
+                       (cd *)p3);
+    HIPCHK(hipGetLastError());
+    HIPCHK(hipStreamSynchronize(e->stream));
+    g.ybase = (const cd *)p3;
+    g.ent = (const cd *)p1;
+    g.ent_fd = (const double2 *)p2;
+  }
   UP(g.Gs, e->Gs); UP(g.Qd, e->Qd); UP(g.Va0, e->Va);
   UP(g.base_type, e->bus_type);
   {
@@ -1508,17 +1535,22 @@ static bpf_status run_fd(bpf_engine *e) {
   return BPF_OK;
 }
 
+static void launch_ybus_changed(bpf_engine *e) {
+  if (e->m)
+    hipLaunchKernelGGL(k_ybus_changed, xgrid(e->T, 4 * (size_t)e->m, 256), dim3(256), 0,
+                       e->stream, e->g, e->d);
+}
+
 static bpf_status solve_once(bpf_engine *e, bool *graph_failed) {
   const bool fd = e->opt.alg != BPF_NR;
   const unsigned T = (unsigned)e->T;
-  tbegin(e, "ybus");
-  hipLaunchKernelGGL(k_ybus, xgrid(T, e->g.nnzY, 256), dim3(256), 0,
-                     e->stream, e->g, e->d);
-  tend(e);
   tbegin(e, "init");
-  hipLaunchKernelGGL(k_init, xgrid(T, e->n, 256), dim3(256), 0,
+  hipLaunchKernelGGL(k_init, xgrid(T, e->g.nnzY, 256), dim3(256), 0,
                      e->stream, e->g, e->d, (const int8_t *)e->d_type0,
-                     (const double *)e->d_Qinj0);
+                     (const double *)e->d_Qinj0, 1);
+  tend(e);
+  tbegin(e, "ybus");
+  launch_ybus_changed(e);
   tend(e);
   launch_mismatch(e, 0);
   HIPCHK(hipMemcpyAsync(e->h_count, e->d.active_count, sizeof(int),
@@ -1530,8 +1562,17 @@ static bpf_status solve_once(bpf_engine *e, bool *graph_failed) {
     if (s || *graph_failed) return s;
   }
   tbegin(e, "loss");
-  hipLaunchKernelGGL(k_loss, dim3(T), dim3(1024), 0, e->stream, e->g, e->d,
-                     e->d_Sf, e->d_St, e->d_loss);
+  const size_t parts = div_up(e->m, 256);
+  if (e->m <= LOSS_ONE || parts > 2 * (size_t)e->S.nb) {
+    hipLaunchKernelGGL(k_loss, dim3(T), dim3(1024), 0, e->stream, e->g, e->d,
+                       e->d_Sf, e->d_St, e->d_loss);
+  } else {
+    // the partial sums in the refinement's right-hand side, free by now
+    hipLaunchKernelGGL(k_flows, xgrid(T, e->m, 256), dim3(256), 0, e->stream, e->g, e->d,
+                       e->d_Sf, e->d_St, e->d.rhs);
+    hipLaunchKernelGGL(k_loss_sum, dim3(T), dim3(64), 0, e->stream, e->d,
+                       (const double *)e->d.rhs, (int)parts, e->d_loss);
+  }
   tend(e);
   HIPCHK(hipStreamSynchronize(e->stream));
   HIPCHK(hipGetLastError());
@@ -1571,6 +1612,7 @@ extern "C" bpf_status bpf_make_ybus(bpf_engine *e) {
   if (e->T <= 0) { e->err = "bpf_set_instances not called"; return BPF_ERR_STATE; }
   hipLaunchKernelGGL(k_ybus, xgrid(e->T, e->g.nnzY, 256), dim3(256), 0,
                      e->stream, e->g, e->d);
+  launch_ybus_changed(e);
   HIPCHK(hipGetLastError());
   HIPCHK(hipStreamSynchronize(e->stream));
   e->ybus_ready = true;
@@ -2217,7 +2259,7 @@ static void fd_index(const bpf_engine *e, const int8_t *ty, int which,
 static bpf_status stage_start(bpf_engine *e, const double *V) {
   hipLaunchKernelGGL(k_init, xgrid(e->T, e->n, 256), dim3(256), 0, e->stream,
                      e->g, e->d, (const int8_t *)e->d_type0,
-                     (const double *)e->d_Qinj0);
+                     (const double *)e->d_Qinj0, 0);
   HIPCHK(hipGetLastError());
   if (V) {
     bpf_status s = bus_rows_upload(e, (const cd *)V, e->d.V, e->T);

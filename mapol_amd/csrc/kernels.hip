@@ -51,14 +51,11 @@ __global__ void k_branch_pre(DevTopo g, cd *ys, cd *ejs) {
   ejs[b] = cexpj(M_PI / 180.0 * g.shift[b]);
 }
 
-// pi-model entry of branch b for instance arrays (makeYbus.h:63-80)
-__device__ cd branch_entry(const DevTopo &g, const DevInst &d, int t, int b,
-                           int kind) {
-  const bool on = d.br_on[(size_t)t * g.m + b] != 0;
+// pi-model entry of branch b in service or not, at a tap (makeYbus.h:63-80)
+__device__ cd branch_entry_at(const DevTopo &g, int b, int kind, bool on, double tp) {
   const double stat = on ? 1.0 : 0.0;
   // stat / (R + jX): the precomputed quotient for an in-service branch
   const cd Ys = on ? g.ys[b] : cdiv(mk(0.0, 0.0), mk(g.R[b], g.X[b]));
-  double tp = d.tap[(size_t)t * g.m + b];
   cd tap = (tp != 0.0) ? mk(tp, 0.0) : mk(1.0, 0.0);
   tap = cmul(tap, g.ejs[b]);
   switch (kind) {
@@ -74,6 +71,33 @@ __device__ cd branch_entry(const DevTopo &g, const DevInst &d, int t, int b,
       return cadd(Ys, cdiv(Bc, mk(2.0, 0.0)));
     }
   }
+}
+
+// the entry for instance t
+__device__ __forceinline__ cd branch_entry(const DevTopo &g, const DevInst &d, int t, int b,
+                                           int kind) {
+  const size_t o = (size_t)t * g.m + b;
+  return branch_entry_at(g, b, kind, d.br_on[o] != 0, d.tap[o]);
+}
+
+// all four; out of the case's table for a branch in service at the case's tap
+// (the divisions of each entry are long, and its loads then wait in turn)
+struct BranchY {
+  cd ff, ft, tf, tt;
+};
+__device__ __forceinline__ BranchY branch_entries(const DevTopo &g, const DevInst &d, int t,
+                                                  int b) {
+  const size_t o = (size_t)t * g.m + b;
+  const bool on = d.br_on[o] != 0;
+  const double tp = d.tap[o], tp0 = g.tap0[b];
+  BranchY y = ((const BranchY *)g.ent)[b];
+  if (!(on && tp == tp0)) {
+    y.ff = branch_entry_at(g, b, KFF, on, tp);
+    y.ft = branch_entry_at(g, b, KFT, on, tp);
+    y.tf = branch_entry_at(g, b, KTF, on, tp);
+    y.tt = branch_entry_at(g, b, KTT, on, tp);
+  }
+  return y;
 }
 
 // ---------------------------------------------------------------------------
@@ -100,37 +124,70 @@ __device__ __forceinline__ int parts_of(int count) {
 }
 
 // ---------------------------------------------------------------------------
-// Ybus assembly with outage masks: one thread per (position, instance).
-// Sum order = the reference's: from-side terms, then to-side terms, then the
-// bus shunt (Cf*Yf + Ct*Yt + Ysh, makeYbus.h:196-266).
+// Ybus assembly with outage masks.  Sum order = the reference's: from-side
+// terms, then to-side terms, then the bus shunt (Cf*Yf + Ct*Yt + Ysh,
+// makeYbus.h:196-266).  An instance differs from its case in a few branches, so
+// the case's own sums (ybase) are copied to every instance, and the positions
+// of a branch whose status or tap differs are then summed anew; two branches
+// that share a position write the same sum.  Summing every position of every
+// instance waited for the chain of its items' loads: 1500 instances of 1354
+// buses 282 us with the start voltages, 120 now, where the 127 MB take 25;
+// 200 of 9241 buses 312, 117 now.
 // ---------------------------------------------------------------------------
+template <class Entry>
+__device__ __forceinline__ cd ybus_sum(const DevTopo &g, int p, const Entry &entry) {
+  cd af = mk(0.0, 0.0), at = mk(0.0, 0.0);
+  for (int q = g.yf_ptr[p]; q < g.yf_ptr[p + 1]; q++) af = cadd(af, entry(g.yf_item[q]));
+  for (int q = g.yt_ptr[p]; q < g.yt_ptr[p + 1]; q++) at = cadd(at, entry(g.yt_item[q]));
+  return cadd(af, at);
+}
+
+__device__ __forceinline__ cd ybus_shunt(const DevTopo &g, const DevInst &d, int t, int p, cd y) {
+  const int i = g.ydiag_bus[p];
+  return i >= 0 ? cadd(y, mk(g.Gs[i], d.Bs[(size_t)t * g.n + i])) : y;
+}
+
+// once per case
+__global__ void k_ybus_base(DevTopo g, cd *ybase) {
+  const int p = blockIdx.x * blockDim.x + threadIdx.x;
+  if (p >= g.nnzY) return;
+  ybase[p] = ybus_sum(g, p, [&](int it) {
+    return branch_entry_at(g, it >> 2, it & 3, g.on0[it >> 2] != 0, g.tap0[it >> 2]);
+  });
+}
+
+__device__ __forceinline__ void ybus_copy(const DevTopo &g, const DevInst &d, int t, int p) {
+  d.Y[(size_t)t * g.nnzY + p] = ybus_shunt(g, d, t, p, g.ybase[p]);
+}
+
 __global__ void k_ybus(DevTopo g, DevInst d) {
   const XSlot sl = xcd_slot(parts_of(g.nnzY));
   const int t = sl.t, p = sl.part * blockDim.x + threadIdx.x;
-  if (t >= d.T || p >= g.nnzY) return;
-  cd af = mk(0.0, 0.0), at = mk(0.0, 0.0);
-  for (int q = g.yf_ptr[p]; q < g.yf_ptr[p + 1]; q++) {
-    int it = g.yf_item[q];
-    af = cadd(af, branch_entry(g, d, t, it >> 2, it & 3));
-  }
-  for (int q = g.yt_ptr[p]; q < g.yt_ptr[p + 1]; q++) {
-    int it = g.yt_item[q];
-    at = cadd(at, branch_entry(g, d, t, it >> 2, it & 3));
-  }
-  cd y = cadd(af, at);
-  int i = g.ydiag_bus[p];
-  if (i >= 0) y = cadd(y, mk(g.Gs[i], d.Bs[(size_t)t * g.n + i]));
-  d.Y[(size_t)t * g.nnzY + p] = y;
+  if (t < d.T && p < g.nnzY) ybus_copy(g, d, t, p);
+}
+
+// (a thread per branch and position)
+__global__ void k_ybus_changed(DevTopo g, DevInst d) {
+  const XSlot sl = xcd_slot(parts_of(4 * g.m));
+  const int t = sl.t, q = sl.part * blockDim.x + threadIdx.x, b = q >> 2;
+  if (t >= d.T || b >= g.m) return;
+  const size_t o = (size_t)t * g.m + b;
+  if ((d.br_on[o] != 0) == (g.on0[b] != 0) && d.tap[o] == g.tap0[b]) return;
+  const int p = g.ybr[q];
+  const cd y = ybus_sum(g, p, [&](int it) { return branch_entry(g, d, t, it >> 2, it & 3); });
+  d.Y[(size_t)t * g.nnzY + p] = ybus_shunt(g, d, t, p, y);
 }
 
 // ---------------------------------------------------------------------------
-// Initial voltage (runpf.h:211-226) and per-solve state reset.
+// Initial voltage (runpf.h:211-226) and per-solve state reset; ybus: the copy
+// of the case's Ybus in the same launch (more threads than buses)
 // ---------------------------------------------------------------------------
 __global__ void k_init(DevTopo g, DevInst d, const int8_t *type0,
-                       const double *Qinj0) {
-  const XSlot sl = xcd_slot(parts_of(g.n));
+                       const double *Qinj0, int ybus) {
+  const XSlot sl = xcd_slot(parts_of(ybus ? g.nnzY : g.n));
   const int t = sl.t, i = sl.part * blockDim.x + threadIdx.x;
   if (t >= d.T) return;
+  if (ybus && i < g.nnzY) ybus_copy(g, d, t, i);
   if (i == 0 && t == 0) *d.active_count = 0;
   if (i == 0) {
     InstState s;
@@ -2570,13 +2627,13 @@ __global__ void k_fd_update(DevTopo g, DevInst d, int part) {
 // one Ybus-style entry of the modified networks behind B' and B''
 // (makeB.h:311-501): B' zeroes line charging, taps and bus shunts (and R for
 // XB); B'' zeroes phase shifts (and R for BX)
-__device__ cd branch_entry_fd(const DevTopo &g, const DevInst &d, int t, int b,
-                              int kind, int which, int zeroR) {
-  double stat = d.br_on[(size_t)t * g.m + b] ? 1.0 : 0.0;
+__device__ cd branch_entry_fd(const DevTopo &g, int b, int kind, int which, int zeroR,
+                              bool on, double tap_now) {
+  double stat = on ? 1.0 : 0.0;
   double R = zeroR ? 0.0 : g.R[b];
   cd Ys = cdiv(mk(stat, 0.0), mk(R, g.X[b]));
   double Bch = (which == 1) ? 0.0 : g.B[b];
-  double tp = (which == 1) ? 0.0 : d.tap[(size_t)t * g.m + b];
+  double tp = (which == 1) ? 0.0 : tap_now;
   double sh = (which == 1) ? g.shift[b] : 0.0;
   cd tap = (tp != 0.0) ? mk(tp, 0.0) : mk(1.0, 0.0);
   tap = cmul(tap, cexpj(M_PI / 180.0 * sh));
@@ -2589,6 +2646,32 @@ __device__ cd branch_entry_fd(const DevTopo &g, const DevInst &d, int t, int b,
   }
 }
 
+__device__ __forceinline__ double2 branch_b_at(const DevTopo &g, int b, int kind, int alg,
+                                               bool on, double tp) {
+  return make_double2(branch_entry_fd(g, b, kind, 1, alg == 1, on, tp).y,
+                      branch_entry_fd(g, b, kind, 2, alg == 2, on, tp).y);
+}
+
+// the imaginary parts {B', B''} of branch b's entry for instance t
+__device__ __forceinline__ double2 branch_b(const DevTopo &g, const DevInst &d, int t, int b,
+                                            int kind, int alg) {
+  const size_t o = (size_t)t * g.m + b;
+  const bool on = d.br_on[o] != 0;
+  const double tp = d.tap[o];
+  if (on && tp == g.tap0[b]) return g.ent_fd[4 * b + kind];
+  return branch_b_at(g, b, kind, alg, on, tp);
+}
+
+// the tables of the branches in service at the case's taps, once per case with
+// the operations an instance's own entries take (ent_fd: decoupled engines)
+__global__ void k_branch_entries(DevTopo g, int alg, cd *ent, double2 *ent_fd) {
+  const int q = blockIdx.x * blockDim.x + threadIdx.x;
+  if (q >= 4 * g.m) return;
+  const int b = q >> 2, kind = q & 3;
+  ent[q] = branch_entry_at(g, b, kind, true, g.tap0[b]);
+  if (ent_fd) ent_fd[q] = branch_b_at(g, b, kind, alg, true, g.tap0[b]);
+}
+
 // B' and B'' of every instance as one block-diagonal 2x2 system in the L+U
 // storage: block (i,j) = [B'_ij 0; 0 B''_ij], with an identity Q row for PV
 // buses; B = -Im(Ybus of the modified network).  alg: 1 XB, 2 BX.
@@ -2598,33 +2681,29 @@ __global__ void k_bmat(DevTopo g, DevInst d, int alg, B4<double> *LU) {
   if (p >= g.nnzY) return;
   int q = g.y2lu[p];
   if (q < 0) return;
-  double v[2];
-  for (int which = 1; which <= 2; which++) {
-    int zeroR = (which == 1 && alg == 1) || (which == 2 && alg == 2);
-    cd af = mk(0.0, 0.0), at = mk(0.0, 0.0);
-    for (int r = g.yf_ptr[p]; r < g.yf_ptr[p + 1]; r++) {
-      int it = g.yf_item[r];
-      af = cadd(af, branch_entry_fd(g, d, t, it >> 2, it & 3, which, zeroR));
-    }
-    for (int r = g.yt_ptr[p]; r < g.yt_ptr[p + 1]; r++) {
-      int it = g.yt_item[r];
-      at = cadd(at, branch_entry_fd(g, d, t, it >> 2, it & 3, which, zeroR));
-    }
-    cd y = cadd(af, at);
-    int i = g.ydiag_bus[p];
-    if (i >= 0) {
-      double bs = (which == 1) ? 0.0 : d.Bs[(size_t)t * g.n + i];
-      y = cadd(y, mk(g.Gs[i], bs));
-    }
-    v[which - 1] = -y.y;
+  double2 f = make_double2(0.0, 0.0), a = make_double2(0.0, 0.0);
+  for (int r = g.yf_ptr[p]; r < g.yf_ptr[p + 1]; r++) {
+    const int it = g.yf_item[r];
+    const double2 y = branch_b(g, d, t, it >> 2, it & 3, alg);
+    f.x += y.x;
+    f.y += y.y;
   }
+  for (int r = g.yt_ptr[p]; r < g.yt_ptr[p + 1]; r++) {
+    const int it = g.yt_item[r];
+    const double2 y = branch_b(g, d, t, it >> 2, it & 3, alg);
+    a.x += y.x;
+    a.y += y.y;
+  }
+  const int i = g.ydiag_bus[p];
+  double v[2] = {f.x + a.x, f.y + a.y};
+  if (i >= 0) v[1] += d.Bs[(size_t)t * g.n + i];
   int ii = g.yrowof[p], jj = g.ycol[p];
   int ti = d.type[(size_t)t * g.n + ii], tj = d.type[(size_t)t * g.n + jj];
   B4<double> blk;
-  blk.a = v[0];
+  blk.a = -v[0];
   blk.b = 0.0;
   blk.c = 0.0;
-  blk.d = (ti == 2 || tj == 2) ? ((ii == jj) ? 1.0 : 0.0) : v[1];
+  blk.d = (ti == 2 || tj == 2) ? ((ii == jj) ? 1.0 : 0.0) : -v[1];
   LU[(size_t)t * g.nnzLU + q] = blk;
 }
 
@@ -2646,10 +2725,11 @@ __device__ BranchState branch_state(const DevTopo &g, const DevInst &d, int t,
   int f = g.br_from[b], to = g.br_to[b];
   s.Vf = V[f];
   s.Vt = V[to];
-  s.yff = branch_entry(g, d, t, b, KFF);
-  s.yft = branch_entry(g, d, t, b, KFT);
-  s.ytf = branch_entry(g, d, t, b, KTF);
-  s.ytt = branch_entry(g, d, t, b, KTT);
+  const BranchY yb = branch_entries(g, d, t, b);
+  s.yff = yb.ff;
+  s.yft = yb.ft;
+  s.ytf = yb.tf;
+  s.ytt = yb.tt;
   cd If = cadd(cmul(s.yff, s.Vf), cmul(s.yft, s.Vt));
   cd It = cadd(cmul(s.ytf, s.Vf), cmul(s.ytt, s.Vt));
   s.Sf = cmul(s.Vf, cconj(If));
@@ -2852,34 +2932,64 @@ __global__ void k_objective(DevTopo g, DevInst d, const double *rate, double w,
 
 // ---------------------------------------------------------------------------
 // Losses and branch flows (computeLoss + reduceLoss, runpf.h:543-604; CPU
-// runpf.h:228-257).  One workgroup per instance.
+// runpf.h:228-257).  A compute unit gathers one line a cycle (four of entries
+// and two of voltages per branch), so one workgroup per instance left the chip
+// idle: up to LOSS_ONE branches k_loss, else k_flows with a workgroup per 256
+// branches and its sum in part, and k_loss_sum (one instance of 9241 buses
+// 51 -> 10 us, 200 of them 92 -> 72; 14 buses would pay a second launch of 4
+// us for nothing).
 // ---------------------------------------------------------------------------
+constexpr int LOSS_ONE = 1024;
+
+__device__ __forceinline__ double branch_flow(const DevTopo &g, const DevInst &d, int t, int b,
+                                              cd *Sf, cd *St) {
+  const int f = g.br_from[b], to = g.br_to[b];
+  const BranchY y = branch_entries(g, d, t, b);
+  const cd *V = d.V + (size_t)t * g.n;
+  const cd vf = V[f], vt = V[to];
+  cd If, It;
+  if (f < to) {
+    If = cadd(cmul(y.ff, vf), cmul(y.ft, vt));
+    It = cadd(cmul(y.tf, vf), cmul(y.tt, vt));
+  } else {
+    If = cadd(cmul(y.ft, vt), cmul(y.ff, vf));
+    It = cadd(cmul(y.tt, vt), cmul(y.tf, vf));
+  }
+  const cd sf = cmul(cconj(If), vf);
+  const cd s2 = cmul(cconj(It), vt);
+  Sf[(size_t)t * g.m + b] = cconj(sf);
+  St[(size_t)t * g.m + b] = cconj(s2);
+  return cadd(sf, s2).x;
+}
+
 __global__ void k_loss(DevTopo g, DevInst d, cd *Sf, cd *St, double *loss) {
   __shared__ double sh[16];
   const int t = blockIdx.x;
-  const cd *V = d.V + (size_t)t * g.n;
   double acc = 0.0;
-  for (int b = threadIdx.x; b < g.m; b += blockDim.x) {
-    int f = g.br_from[b], to = g.br_to[b];
-    cd yff = branch_entry(g, d, t, b, KFF), yft = branch_entry(g, d, t, b, KFT);
-    cd ytf = branch_entry(g, d, t, b, KTF), ytt = branch_entry(g, d, t, b, KTT);
-    cd If, It;
-    if (f < to) {
-      If = cadd(cmul(yff, V[f]), cmul(yft, V[to]));
-      It = cadd(cmul(ytf, V[f]), cmul(ytt, V[to]));
-    } else {
-      If = cadd(cmul(yft, V[to]), cmul(yff, V[f]));
-      It = cadd(cmul(ytt, V[to]), cmul(ytf, V[f]));
-    }
-    cd sf = cmul(cconj(If), V[f]);
-    cd s2 = cmul(cconj(It), V[to]);
-    Sf[(size_t)t * g.m + b] = cconj(sf);
-    St[(size_t)t * g.m + b] = cconj(s2);
-    acc += cadd(sf, s2).x;
-  }
+  for (int b = threadIdx.x; b < g.m; b += blockDim.x) acc += branch_flow(g, d, t, b, Sf, St);
   double tot = block_sum(acc, sh);
   if (threadIdx.x == 0)
     loss[t] = (d.st[t].verdict == BPF_V_CONVERGED) ? tot : DBL_MAX;
+}
+
+__global__ void k_flows(DevTopo g, DevInst d, cd *Sf, cd *St, double *part) {
+  __shared__ double sh[16];
+  const int parts = parts_of(g.m);
+  const XSlot sl = xcd_slot(parts);
+  const int t = sl.t, b = sl.part * blockDim.x + threadIdx.x;
+  if (t >= d.T) return;
+  const double tot = block_sum(b < g.m ? branch_flow(g, d, t, b, Sf, St) : 0.0, sh);
+  if (threadIdx.x == 0) part[(size_t)t * parts + sl.part] = tot;
+}
+
+// one wave per instance
+__global__ void k_loss_sum(DevInst d, const double *part, int parts, double *loss) {
+  const int t = blockIdx.x;
+  double acc = 0.0;
+  for (int q = threadIdx.x; q < parts; q += 64) acc += part[(size_t)t * parts + q];
+  acc = wave_sum(acc);
+  if (threadIdx.x == 0)
+    loss[t] = (d.st[t].verdict == BPF_V_CONVERGED) ? acc : DBL_MAX;
 }
 
 // ---------------------------------------------------------------------------

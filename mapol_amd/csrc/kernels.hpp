@@ -42,6 +42,15 @@ struct DevTopo {
   const int *br_from, *br_to, *bbr_ptr, *bbr;
   const double *R, *X, *B, *shift, *Gs, *Qd, *Va0;
   const cd *ys, *ejs;      // per branch: 1 / (R + jX), e^(j shift) (k_branch_pre)
+  // per branch, in service at the case's tap (tap0): its four pi-model entries
+  // and {B', B''} = the imaginary parts of the decoupled networks' entries
+  // (k_branch_entries)
+  const cd *ent;
+  const double2 *ent_fd;
+  const double *tap0;
+  const uint8_t *on0;      // the case's branch status
+  const int *ybr;          // per branch: Ybus positions of its ff, ft, tf, tt entries
+  const cd *ybase;         // Ybus of the case's own branches (no shunts)
   const int *base_type;
   // Jacobian blocks in L+U position order: position, Ybus position
   int nJb;
