@@ -1494,6 +1494,17 @@ static bpf_status run_newton(bpf_engine *e, bool *graph_failed) {
 // assembled and factored once in FP64, then P and Q half-steps; each half-step
 // is a masked solve with the same factors, an update and the |V|-normalised
 // mismatch with the reference's convergence checks
+// The whole decoupled loop in one launch (k_fd_one), a workgroup and compute
+// unit per instance: not for so many buses that their mismatch needs more than
+// one compute unit, nor for many small instances, which the launches keep
+// several to a compute unit.  A solve, launches / one: 14 buses x 1 432 / 158
+// us, 118 x 1 838 / 436, 118 x 2000 3979 / 4265, 1354 x 1 817 / 678, x 200
+// 1508 / 1173, x 1000 4683 / 4087, 2869 x 100 1613 / 1560, 9241 x 1 2025 /
+// 2881, x 200 7023 / 8060.
+static bool fd_one(const bpf_engine *e) {
+  return e->n <= 4096 && (e->n >= 1024 || e->T <= 4 * e->num_cu);
+}
+
 static bpf_status run_fd(bpf_engine *e) {
   B4<double> *LU, *TLd;
   double *xg;
@@ -1509,13 +1520,18 @@ static bpf_status run_fd(bpf_engine *e) {
   tend(e);
   size_t xs = sizeof(double) * 2 * (size_t)e->S.nb;
   int use_lds = xs <= (size_t)SOLVE_LDS_BYTES;
+  const int ep = sweep_mode(e->S, sizeof(double), use_lds, e->sweep_form, e->solve_threads);
+  if (!e->timing && e->solve_threads == 1024 && slot_lanes(e, ep) == 1 && fd_one(e)) {
+    hipLaunchKernelGGL(k_fd_one, dim3(T), dim3(1024), 0, e->stream, e->g, e->d,
+                       (const B4<double> *)LU, (const B4<double> *)TLd, e->splan,
+                       e->opt.maxit_fd, e->opt.tol, e->opt.qlim_tol);
+    HIPCHK(hipGetLastError());
+    return BPF_OK;
+  }
   for (int it = 0; it < e->opt.maxit_fd + 1; it++) {
     for (int half = 1; half <= 2; half++) {
       tbegin(e, "fd_solve");
-      launch_solve<double>(e, T, LU, half, 0, use_lds,
-                           sweep_mode(e->S, sizeof(double), use_lds,
-                                      e->sweep_form, e->solve_threads),
-                           TLd, xg);
+      launch_solve<double>(e, T, LU, half, 0, use_lds, ep, TLd, xg);
       tend(e);
       tbegin(e, "update");
       hipLaunchKernelGGL(k_fd_update, xgrid(T, e->n, 256), dim3(256),

@@ -426,28 +426,13 @@ __global__ void k_mismatch_mb(DevTopo g, DevInst d, int mode, int fd_norm,
   }
 }
 
-__global__ void k_verdict(DevTopo g, DevInst d, int nparts, int mode, int maxit,
-                          double tol, int enforce_qlim, int max_rounds,
-                          double qtol, int fd_norm) {
-  __shared__ double shd[16];
-  __shared__ int shi[16];
-  const int t = blockIdx.x;
-  InstState *sp = d.st + t;
-  if (mode != 2 && sp->done) return;
-  double pm = 0.0;
-  int pn = 0, pv = 0;
-  for (int q = threadIdx.x; q < nparts; q += blockDim.x) {
-    double v = d.part[(size_t)t * nparts + q];
-    pn |= isnan(v);
-    pm = fmax(pm, v);
-    pv += d.partv[(size_t)t * nparts + q];
-  }
-  double nrm = block_max(pm, shd);
-  int anynan = block_or(pn, shi);
-  // PV buses beyond their reactive limits at this V (counted per bus by the
-  // mismatch kernel); after a switch the remaining ones are recounted here
-  int nviol_at_v = enforce_qlim ? block_add(pv, shi) : 0;
-  InstState s = *sp;
+// the decision on a norm (every thread of the instance's workgroup, with the
+// same arguments): the next state, and whether the instance goes on
+__device__ __forceinline__ bool verdict_of(const DevTopo &g, const DevInst &d, int t, double nrm,
+                                           int anynan, int nviol_at_v, int mode, int maxit,
+                                           double tol, int enforce_qlim, int max_rounds,
+                                           double qtol, int fd_norm, double *shd, int *shi,
+                                           InstState &s) {
   if (mode == 1 || mode == 3) { s.it_round++; s.it_total++; }
   int8_t *ty = d.type + (size_t)t * g.n;
   double *Qinj = d.Qinj + (size_t)t * g.n;
@@ -507,6 +492,33 @@ __global__ void k_verdict(DevTopo g, DevInst d, int nparts, int mode, int maxit,
     active = true;
     break;
   }
+  return active;
+}
+
+__global__ void k_verdict(DevTopo g, DevInst d, int nparts, int mode, int maxit,
+                          double tol, int enforce_qlim, int max_rounds,
+                          double qtol, int fd_norm) {
+  __shared__ double shd[16];
+  __shared__ int shi[16];
+  const int t = blockIdx.x;
+  InstState *sp = d.st + t;
+  if (mode != 2 && sp->done) return;
+  double pm = 0.0;
+  int pn = 0, pv = 0;
+  for (int q = threadIdx.x; q < nparts; q += blockDim.x) {
+    double v = d.part[(size_t)t * nparts + q];
+    pn |= isnan(v);
+    pm = fmax(pm, v);
+    pv += d.partv[(size_t)t * nparts + q];
+  }
+  double nrm = block_max(pm, shd);
+  int anynan = block_or(pn, shi);
+  // PV buses beyond their reactive limits at this V (counted per bus by the
+  // mismatch kernel); after a switch the remaining ones are recounted here
+  int nviol_at_v = enforce_qlim ? block_add(pv, shi) : 0;
+  InstState s = *sp;
+  const bool active = verdict_of(g, d, t, nrm, anynan, nviol_at_v, mode, maxit, tol, enforce_qlim,
+                                 max_rounds, qtol, fd_norm, shd, shi, s);
   if (threadIdx.x == 0) {
     *sp = s;
     if (active) atomicAdd(d.active_count, 1);
@@ -2607,11 +2619,8 @@ __global__ void k_count_active(DevInst d) {
 // Fast decoupled: half-step updates (fdpf.h:416-448).  part 1: angles of all
 // unknown buses, part 2: magnitudes of PQ buses.
 // ---------------------------------------------------------------------------
-__global__ void k_fd_update(DevTopo g, DevInst d, int part) {
-  const XSlot sl = xcd_slot(parts_of(g.n));
-  const int t = sl.t, i = sl.part * blockDim.x + threadIdx.x;
-  if (t >= d.T || i >= g.n) return;
-  if (d.st[t].done) return;
+__device__ __forceinline__ void fd_update_bus(const DevTopo &g, const DevInst &d, int t, int i,
+                                              int part) {
   const int k = g.blk_of_bus[i];
   if (k < 0) return;
   size_t o = (size_t)t * g.n + i;
@@ -2622,6 +2631,14 @@ __global__ void k_fd_update(DevTopo g, DevInst d, int part) {
   } else if (d.type[o] == 1) {
     d.V[o] = cmul(mk(cabs_(v) - dx[2 * k + 1], 0.0), cexpj(atan(v.y / v.x)));
   }
+}
+
+__global__ void k_fd_update(DevTopo g, DevInst d, int part) {
+  const XSlot sl = xcd_slot(parts_of(g.n));
+  const int t = sl.t, i = sl.part * blockDim.x + threadIdx.x;
+  if (t >= d.T || i >= g.n) return;
+  if (d.st[t].done) return;
+  fd_update_bus(g, d, t, i, part);
 }
 
 // one Ybus-style entry of the modified networks behind B' and B''
@@ -3063,6 +3080,66 @@ __global__ void k_results(DevInst d, const double *loss, const int *map, int n, 
     st[q] = d.st[q];
     ls[q] = loss[q];
   }
+}
+
+// ---------------------------------------------------------------------------
+// One workgroup runs an instance's whole solve: the steps of an iteration meet
+// at barriers instead of launches, and an instance ends with its own last
+// iteration.  The mismatch of every bus, its norm and the verdict:
+// ---------------------------------------------------------------------------
+__device__ __forceinline__ bool mismatch_verdict(const DevTopo &g, const DevInst &d, int t,
+                                                 int mode, int maxit, double tol, int qlim,
+                                                 int max_rounds, double qtol, int fd_norm,
+                                                 double *shd, int *shi, InstState &s) {
+  double lmax = 0.0;
+  int lnan = 0, lviol = 0;
+  for (int i = threadIdx.x; i < g.n; i += blockDim.x)
+    mis_bus(g, d, t, i, fd_norm, qtol, qlim, lmax, lnan, lviol);
+  const double nrm = block_max(lmax, shd);
+  const int anynan = block_or(lnan, shi);
+  const int nviol = qlim ? block_add(lviol, shi) : 0;
+  return verdict_of(g, d, t, nrm, anynan, nviol, mode, maxit, tol, qlim, max_rounds, qtol, fd_norm,
+                    shd, shi, s);
+}
+
+// the state of an instance that ends, and one active instance less
+__device__ __forceinline__ void finish(const DevInst &d, int t, const InstState &s) {
+  if (threadIdx.x == 0) {
+    d.st[t] = s;
+    if (s.done) atomicSub(d.active_count, 1);
+  }
+}
+
+// Fast decoupled: the P and Q half-steps of every iteration (slot form of the
+// sweeps, X in LDS).  A half-step by launches was five of them and a wait of
+// the host, 72 us at 1354 buses x 200 of which the sweeps take 33; here 48.
+__global__ void __launch_bounds__(1024)
+k_fd_one(DevTopo g, DevInst d, const B4<double> *LU, const B4<double> *TL, SolvePlan P,
+         int maxit, double tol, double qtol) {
+  __shared__ double smem[SOLVE_LDS_BYTES / sizeof(double)];
+  __shared__ double rs[2 * TAIL_MAX];
+  __shared__ int4 s_swc[MAX_CHUNKS];
+  __shared__ double shd[16];
+  __shared__ int shi[16];
+  const int t = blockIdx.x;
+  InstState s = d.st[t];
+  if (s.done) return;
+  const B4<double> *A = LU + (size_t)t * g.nnzLU;
+  const B4<double> *Ti = TL + (size_t)t * P.tn * P.tn;
+  for (int q = threadIdx.x; q < P.sl_nfw + P.sl_nbw; q += blockDim.x) s_swc[q] = P.sl_chunk[q];
+  if (threadIdx.x < SLOT_X_PAD) smem[threadIdx.x] = 0.0;
+  for (int it = 0; it < 2 * (maxit + 1); it++) {
+    const int half = 1 + (it & 1);
+    solve_pass<double, true, 1>(g, A, Ti, smem + SLOT_X_PAD, nullptr, rs, s_swc, nullptr, P, 0,
+                                d.F + (size_t)t * 2 * g.nb, half, 0,
+                                d.dx + (size_t)t * 2 * g.nb);
+    __syncthreads();
+    for (int i = threadIdx.x; i < g.n; i += blockDim.x) fd_update_bus(g, d, t, i, half);
+    __syncthreads();
+    if (!mismatch_verdict(g, d, t, half == 1 ? 3 : 4, maxit, tol, 0, 0, qtol, 1, shd, shi, s)) break;
+    __syncthreads();
+  }
+  finish(d, t, s);
 }
 
 // explicit instantiations used by the engine
