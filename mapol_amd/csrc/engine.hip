@@ -1373,7 +1373,22 @@ struct PartScope {
   }
 };
 
-static bpf_status run_newton(bpf_engine *e, bool *graph_failed) {
+// branch flows and losses; gate and count: loss_waits
+static void launch_loss(bpf_engine *e, const int *gate, int *count) {
+  const size_t parts = div_up(e->m, 256);
+  if (e->m <= LOSS_ONE || parts > 2 * (size_t)e->S.nb) {
+    hipLaunchKernelGGL(k_loss, dim3(e->T), dim3(1024), 0, e->stream, e->g, e->d,
+                       e->d_Sf, e->d_St, e->d_loss, gate, count);
+  } else {
+    // the partial sums in the refinement's right-hand side, free by now
+    hipLaunchKernelGGL(k_flows, xgrid(e->T, e->m, 256), dim3(256), 0, e->stream, e->g, e->d,
+                       e->d_Sf, e->d_St, e->d.rhs, gate);
+    hipLaunchKernelGGL(k_loss_sum, dim3(e->T), dim3(64), 0, e->stream, e->d,
+                       (const double *)e->d.rhs, (int)parts, e->d_loss, gate, count);
+  }
+}
+
+static bpf_status run_newton(bpf_engine *e, bool *graph_failed, bool *loss_done) {
   bpf_status s = ensure_lu(e, e->opt.precision == BPF_FP64 ? 1 : 0);
   if (s) return s;
   // per-kernel timing uses events around direct launches: elapsed times
@@ -1442,7 +1457,12 @@ static bpf_status run_newton(bpf_engine *e, bool *graph_failed) {
         if (!active[h]) continue;
         where = "hipGraphLaunch";
         r = hipGraphLaunch(*slot[h], view[h].s);
-        if (r == hipSuccess) {
+        if (r == hipSuccess && K == 1) {
+          // the losses behind the replay: they are summed if it was the last
+          // one, and their kernel hands the count to the host (a wait less
+          // per solve, and a copy less per replay)
+          launch_loss(e, e->d.active_count, e->h_count);
+        } else if (r == hipSuccess) {
           where = "hipMemcpyAsync";
           r = hipMemcpyAsync(view[h].hc, view[h].d.active_count, sizeof(int),
                              hipMemcpyDeviceToHost, view[h].s);
@@ -1485,7 +1505,10 @@ static bpf_status run_newton(bpf_engine *e, bool *graph_failed) {
       active[h] = active[h] && view[h].hc[0] > 0;
       any = any || active[h];
     }
-    if (!any) break;
+    if (!any) {
+      *loss_done = use_graph && K == 1;
+      break;
+    }
   }
   return BPF_OK;
 }
@@ -1569,28 +1592,26 @@ static bpf_status solve_once(bpf_engine *e, bool *graph_failed) {
   launch_ybus_changed(e);
   tend(e);
   launch_mismatch(e, 0);
-  HIPCHK(hipMemcpyAsync(e->h_count, e->d.active_count, sizeof(int),
-                        hipMemcpyDeviceToHost, e->stream));
-  HIPCHK(hipStreamSynchronize(e->stream));
-  HIPCHK(hipGetLastError());
-  if (*e->h_count > 0) {
-    bpf_status s = fd ? run_fd(e) : run_newton(e, graph_failed);
+  // a replayed iteration leaves a batch without active instances alone, so the
+  // first replay is queued without waiting for the count
+  bool loss_done = false;
+  const bool queue = !fd && e->opt.use_graph && !e->graph_broken && !e->timing;
+  if (!queue) {
+    HIPCHK(hipMemcpyAsync(e->h_count, e->d.active_count, sizeof(int),
+                          hipMemcpyDeviceToHost, e->stream));
+    HIPCHK(hipStreamSynchronize(e->stream));
+    HIPCHK(hipGetLastError());
+  }
+  if (queue || *e->h_count > 0) {
+    bpf_status s = fd ? run_fd(e) : run_newton(e, graph_failed, &loss_done);
     if (s || *graph_failed) return s;
   }
-  tbegin(e, "loss");
-  const size_t parts = div_up(e->m, 256);
-  if (e->m <= LOSS_ONE || parts > 2 * (size_t)e->S.nb) {
-    hipLaunchKernelGGL(k_loss, dim3(T), dim3(1024), 0, e->stream, e->g, e->d,
-                       e->d_Sf, e->d_St, e->d_loss);
-  } else {
-    // the partial sums in the refinement's right-hand side, free by now
-    hipLaunchKernelGGL(k_flows, xgrid(T, e->m, 256), dim3(256), 0, e->stream, e->g, e->d,
-                       e->d_Sf, e->d_St, e->d.rhs);
-    hipLaunchKernelGGL(k_loss_sum, dim3(T), dim3(64), 0, e->stream, e->d,
-                       (const double *)e->d.rhs, (int)parts, e->d_loss);
+  if (!loss_done) {
+    tbegin(e, "loss");
+    launch_loss(e, nullptr, nullptr);
+    tend(e);
+    HIPCHK(hipStreamSynchronize(e->stream));
   }
-  tend(e);
-  HIPCHK(hipStreamSynchronize(e->stream));
   HIPCHK(hipGetLastError());
   return BPF_OK;
 }

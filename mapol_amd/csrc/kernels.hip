@@ -2979,9 +2979,20 @@ __device__ __forceinline__ double branch_flow(const DevTopo &g, const DevInst &d
   return cadd(sf, s2).x;
 }
 
-__global__ void k_loss(DevTopo g, DevInst d, cd *Sf, cd *St, double *loss) {
+// gate (or null): the batch's count of active instances, passed on to the host's
+// count; while it isn't zero the solve goes on and there is nothing to sum
+__device__ __forceinline__ bool loss_waits(const int *gate, int *count) {
+  if (!gate) return false;
+  const int a = *gate;
+  if (count && blockIdx.x == 0 && threadIdx.x == 0) *count = a;
+  return a != 0;
+}
+
+__global__ void k_loss(DevTopo g, DevInst d, cd *Sf, cd *St, double *loss, const int *gate,
+                       int *count) {
   __shared__ double sh[16];
   const int t = blockIdx.x;
+  if (loss_waits(gate, count)) return;
   double acc = 0.0;
   for (int b = threadIdx.x; b < g.m; b += blockDim.x) acc += branch_flow(g, d, t, b, Sf, St);
   double tot = block_sum(acc, sh);
@@ -2989,8 +3000,9 @@ __global__ void k_loss(DevTopo g, DevInst d, cd *Sf, cd *St, double *loss) {
     loss[t] = (d.st[t].verdict == BPF_V_CONVERGED) ? tot : DBL_MAX;
 }
 
-__global__ void k_flows(DevTopo g, DevInst d, cd *Sf, cd *St, double *part) {
+__global__ void k_flows(DevTopo g, DevInst d, cd *Sf, cd *St, double *part, const int *gate) {
   __shared__ double sh[16];
+  if (loss_waits(gate, nullptr)) return;
   const int parts = parts_of(g.m);
   const XSlot sl = xcd_slot(parts);
   const int t = sl.t, b = sl.part * blockDim.x + threadIdx.x;
@@ -3000,8 +3012,10 @@ __global__ void k_flows(DevTopo g, DevInst d, cd *Sf, cd *St, double *part) {
 }
 
 // one wave per instance
-__global__ void k_loss_sum(DevInst d, const double *part, int parts, double *loss) {
+__global__ void k_loss_sum(DevInst d, const double *part, int parts, double *loss,
+                           const int *gate, int *count) {
   const int t = blockIdx.x;
+  if (loss_waits(gate, count)) return;
   double acc = 0.0;
   for (int q = threadIdx.x; q < parts; q += 64) acc += part[(size_t)t * parts + q];
   acc = wave_sum(acc);
