@@ -169,6 +169,7 @@ struct bpf_engine {
   bool fplan_split = false;
   int split_mode = 0;
   bool fused_set = false;            // bpf_set_fused_forward was called
+  bool solve_set = false;            // bpf_set_launch chose the solve's lanes
   int num_cu = 256;
   int parts_running = 1;
   bool capturing = false;            // recording the iteration graph
@@ -853,7 +854,10 @@ extern "C" bpf_status bpf_set_launch(bpf_engine *e, int32_t lu, int32_t sv,
     return BPF_ERR_INVALID_ARG;
   }
   if (lu) e->lu_threads = lu;
-  if (sv) e->solve_threads = sv;
+  if (sv) {
+    e->solve_threads = sv;
+    e->solve_set = true;
+  }
   if (mis) e->mis_threads = mis;
   drop_graphs(e);
   return BPF_OK;
@@ -1157,11 +1161,28 @@ static void launch_mismatch(bpf_engine *e, int mode) {
   tend(e);
 }
 
+// Lanes of a solve's workgroup, unless the caller chose them.  1024 lanes fill a
+// compute unit with one instance; with more instances than compute units the
+// slot form takes 256 and four slots a lane where three such workgroups fit the
+// LDS, and the chunks' barriers and round trips of several instances overlap.
+// A pass, 1024 / 256 lanes: 1354 buses x 200 26 / 32 us, x 400 47 / 35, x 1500
+// 153 / 91, in FP64 164 / 141; 2869 x 600 110 / 87; 118 x 2000 64 / 41; 9241 x
+// 600, one workgroup either way, 321 / 454.
+static int solve_lanes(const bpf_engine *e, size_t scalar) {
+  const size_t xs = scalar * 2 * (size_t)e->S.nb, lds = xs + SOLVE_LDS_FIXED;
+  return !e->solve_set && e->solve_threads == 1024 &&
+                 e->T * std::max(1, e->parts_running) > e->num_cu &&
+                 3 * lds <= (size_t)160 * 1024 && e->S.prm.slot_chunk <= 1024 &&
+                 sweep_mode(e->S, scalar, 1, e->sweep_form, 1024) == 2
+             ? 256
+             : e->solve_threads;
+}
+
 // slots per lane of the slot form's kernel (0: another form runs)
-static int slot_lanes(const bpf_engine *e, int ep) {
+static int slot_lanes(const bpf_engine *e, int ep, int threads) {
   int sp = 1;
-  while (sp < 8 && sp * e->solve_threads < e->S.prm.slot_chunk) sp *= 2;
-  return ep == 2 && sp * e->solve_threads >= e->S.prm.slot_chunk ? sp : 0;
+  while (sp < 8 && sp * threads < e->S.prm.slot_chunk) sp *= 2;
+  return ep == 2 && sp * threads >= e->S.prm.slot_chunk ? sp : 0;
 }
 
 // one sweep pass of k_lu_solve; the slot form (ep 2) has one kernel per
@@ -1171,16 +1192,22 @@ template <typename T>
 static void launch_solve(bpf_engine *e, int T_, const void *LU, int rhs_mode,
                          int accumulate, int use_lds, int ep,
                          const void *TL = nullptr, void *xglob = nullptr) {
-  const int th = e->solve_threads;
+  const int th = solve_lanes(e, sizeof(T));
   if (!TL) { TL = e->d_TL; xglob = e->d_xglob; }
   SolvePlan sp_ = e->splan;
   sp_.fused_limit = e->fused_forward;     // as the factorization of this step
+  // LDS for what the form keeps there (nothing for X in global memory)
+  const size_t nx = ep == 2   ? 2 * (size_t)e->S.nb + SLOT_X_PAD
+                    : ep == 1 ? (size_t)ep_offset(e->S.nb) + 2 * (size_t)SWEEP_CHUNK
+                    : use_lds ? 2 * (size_t)e->S.nb
+                              : 0;
+  const size_t lds = (sizeof(T) * nx + 15) / 16 * 16;
   auto go = [&](auto kern) {
-    hipLaunchKernelGGL(kern, dim3(T_), dim3(th), 0, e->stream, e->g, e->d,
+    hipLaunchKernelGGL(kern, dim3(T_), dim3(th), lds, e->stream, e->g, e->d,
                        (const B4<T> *)LU, (const B4<T> *)TL, rhs_mode,
                        accumulate, sp_, use_lds, ep, (T *)xglob);
   };
-  const int sp = slot_lanes(e, ep);
+  const int sp = slot_lanes(e, ep, th);
   if (sp > 0) {
     if (sp == 1) go(k_lu_solve<T, 1>);
     else if (sp == 2) go(k_lu_solve<T, 2>);
@@ -1233,12 +1260,13 @@ static void launch_newton_step(bpf_engine *e) {
   const int c0 = e->S.l0_chunks;
   size_t xs = sizeof(T) * 2 * (size_t)e->S.nb;
   int use_lds = xs <= (size_t)SOLVE_LDS_BYTES;
-  const int ep = sweep_mode(e->S, sizeof(T), use_lds, e->sweep_form, e->solve_threads);
+  const int th = solve_lanes(e, sizeof(T));
+  const int ep = sweep_mode(e->S, sizeof(T), use_lds, e->sweep_form, th);
   // with the slot-form sweeps the factorization can also form the forward
   // substitution of the mismatch (the fill writes its right-hand side, and
   // the first solve starts from it; the kernels leave it out while more
   // than the plan's limit of instances are active)
-  const int fused = slot_lanes(e, ep) > 0 && e->fplan.fused_limit >= 0 ? 1 : 0;
+  const int fused = slot_lanes(e, ep, th) > 0 && e->fplan.fused_limit >= 0 ? 1 : 0;
   FactorPlan fp = e->fplan;
   if (!fused) fp.fused_limit = -1;
   const bool resident = resident_runs(e, sizeof(T) == 8);
@@ -1544,7 +1572,7 @@ static bpf_status run_fd(bpf_engine *e) {
   size_t xs = sizeof(double) * 2 * (size_t)e->S.nb;
   int use_lds = xs <= (size_t)SOLVE_LDS_BYTES;
   const int ep = sweep_mode(e->S, sizeof(double), use_lds, e->sweep_form, e->solve_threads);
-  if (!e->timing && e->solve_threads == 1024 && slot_lanes(e, ep) == 1 && fd_one(e)) {
+  if (!e->timing && e->solve_threads == 1024 && slot_lanes(e, ep, 1024) == 1 && fd_one(e)) {
     hipLaunchKernelGGL(k_fd_one, dim3(T), dim3(1024), 0, e->stream, e->g, e->d,
                        (const B4<double> *)LU, (const B4<double> *)TLd, e->splan,
                        e->opt.maxit_fd, e->opt.tol, e->opt.qlim_tol);
@@ -2232,7 +2260,7 @@ extern "C" bpf_status bpf_adjoint(bpf_engine *e, const double *rate, double w,
   hipLaunchKernelGGL(k_jacobian<double>, xgrid(TT, ((size_t)e->g.nJb + 1) / 2, 256),
                      dim3(256), 0, e->stream, e->g, e->d, LU, 0, -1);
   factor_fp64(e, LU, TLd);
-  hipLaunchKernelGGL(k_adj_rhs, dim3(div_up(e->S.nb, 256), TT), dim3(256), 0,
+  hipLaunchKernelGGL(k_adj_rhs, dim3(div_up(4 * (size_t)e->S.nb, 256), TT), dim3(256), 0,
                      e->stream, e->g, e->d, d_rate, w, a.G);
   size_t xs = sizeof(double) * nb2;
   int use_lds = xs <= (size_t)SOLVE_LDS_BYTES;
@@ -2255,7 +2283,7 @@ extern "C" bpf_status bpf_adjoint(bpf_engine *e, const double *rate, double w,
   hipLaunchKernelGGL(k_adj_grad, dim3(div_up(std::max(n, m), 256), TT),
                      dim3(256), 0, e->stream, e->g, e->d,
                      (const double *)a.lam, d_rate, w, a.gP, a.gQ, a.gx);
-  hipLaunchKernelGGL(k_objective, dim3(TT), dim3(256), 0, e->stream, e->g,
+  hipLaunchKernelGGL(k_objective, dim3(TT), dim3(1024), 0, e->stream, e->g,
                      e->d, d_rate, w, a.obj);
   tend(e);
   // factorization singularities are not expected at a converged point; keep

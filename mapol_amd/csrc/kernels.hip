@@ -2394,6 +2394,8 @@ __device__ __forceinline__ void lu_sweeps_slot(const B4<T> *A, const B4<T> *Ti,
 constexpr int SOLVE_LDS_BYTES = 148 * 1024;
 // the slot form keeps a zero pair before X (the x of slots without an entry)
 constexpr int SLOT_X_PAD = 2;
+// k_lu_solve's other LDS: chunk tables and the tail's right-hand side
+constexpr int SOLVE_LDS_FIXED = MAX_CHUNKS * 20 + 2 * TAIL_MAX * 8 + 64;
 // the entry-parallel sweeps keep their product buffer (2 * SWEEP_CHUNK
 // scalars) after X in the same LDS block
 __host__ __device__ constexpr int ep_offset(int nb) { return (2 * nb + 3) & ~3; }
@@ -2473,11 +2475,15 @@ __device__ __forceinline__ void solve_pass(const DevTopo &g, const B4<T> *A,
 // workgroup's lanes (the launch bound lets the larger slot counts of
 // narrower workgroups stay in registers)
 template <typename T, int SP>
+// (held to 128 registers for a fourth workgroup of 256 lanes, FP32 spills 16:
+// 1354 buses x 1500 116 us for 91)
 __global__ void __launch_bounds__(SP > 0 && SLOT_CHUNK / SP < 1024 ? SLOT_CHUNK / SP : 1024)
 k_lu_solve(DevTopo g, DevInst d, const B4<T> *LU, const B4<T> *TL,
            int rhs_mode, int accumulate, SolvePlan P, int use_lds, int ep,
            T *xglob) {
-  __shared__ T smem[SOLVE_LDS_BYTES / sizeof(T)];
+  // X (and the product buffer of the entry-parallel form)
+  extern __shared__ __align__(16) char solve_lds[];
+  T *const smem = (T *)solve_lds;
   __shared__ T rs[2 * TAIL_MAX];
   // the chunk table in LDS (see the factorization)
   __shared__ int4 s_swc[MAX_CHUNKS];
@@ -2766,13 +2772,16 @@ __device__ BranchState branch_state(const DevTopo &g, const DevInst &d, int t,
 // right-hand side G = df/dx in block order (angle, magnitude of PQ buses)
 __global__ void k_adj_rhs(DevTopo g, DevInst d, const double *rate, double w,
                           double *G) {
-  int k = blockIdx.x * blockDim.x + threadIdx.x;
+  // four lanes per bus share its branches: a branch is a chain of loads and
+  // long FP64 operations, and a bus alone waited for all of its own (32
+  // instances of 2869 buses 28 -> 17 us)
+  const int x = blockIdx.x * blockDim.x + threadIdx.x, k = x >> 2, part = x & 3;
   int t = blockIdx.y;
   if (k >= g.nb) return;
   if (d.st[t].done) return;
   int i = g.bus_of_blk[k];
   double ga = 0.0, gm = 0.0;
-  for (int q = g.bbr_ptr[i]; q < g.bbr_ptr[i + 1]; q++) {
+  for (int q = g.bbr_ptr[i] + part; q < g.bbr_ptr[i + 1]; q += 4) {
     int b = g.bbr[q];
     BranchState s = branch_state(g, d, t, b, rate, w);
     cd dSf_a, dSt_a, dSf_m, dSt_m;
@@ -2793,6 +2802,12 @@ __global__ void k_adj_rhs(DevTopo g, DevInst d, const double *rate, double w,
     ga += cmul(s.af, dSf_a).x + cmul(s.at, dSt_a).x;
     gm += cmul(s.af, dSf_m).x + cmul(s.at, dSt_m).x;
   }
+#pragma unroll
+  for (int o = 1; o < 4; o *= 2) {
+    ga += __shfl_xor(ga, o, 64);
+    gm += __shfl_xor(gm, o, 64);
+  }
+  if (part) return;
   double *Gt = G + (size_t)t * 2 * g.nb;
   Gt[2 * k] = ga;
   Gt[2 * k + 1] = (d.type[(size_t)t * g.n + i] == 1) ? gm : 0.0;

@@ -58,3 +58,28 @@ def test_adjoint_at_every_chunk_length(slot_chunk):
     e.close()
     for k in ("grad_P", "grad_Q", "grad_x"):
         assert np.abs(got[k] - ref[k]).max() <= 1e-9 * np.abs(ref[k]).max(), k
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("precision", [0, 1])
+@pytest.mark.parametrize("name,T", [("pf118x200", 256), ("pf118x200", 257), ("pf1354x200", 257),
+                                    ("pf2869x100", 257)])
+def test_solve_lanes_by_instance_count(name, T, precision):
+    """either side of the instance count where the solve takes narrower
+    workgroups, against the wide ones: one order of sums, so the counts are
+    equal and voltages of a quadratic convergence agree to 1e-9"""
+    case, cont = synth.workload(name, T=T)
+    out = []
+    for lanes in (0, 1024):
+        e = engine.Engine(case, precision=precision)
+        if lanes:
+            e.set_launch(solve=lanes)
+        e.set_instances(br_on=cont.br_on, gen_on=cont.gen_on)
+        e.solve()
+        out.append(e.results())
+        e.close()
+    for k in ("iterations", "verdict"):
+        np.testing.assert_array_equal(out[0][k], out[1][k])
+    ok = out[1]["verdict"] == 0
+    assert ok.sum() > T // 2
+    assert np.abs(out[0]["V"][ok] - out[1]["V"][ok]).max() <= 1e-9
