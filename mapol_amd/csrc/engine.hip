@@ -1147,8 +1147,10 @@ static void mismatch_pair(bpf_engine *e, int mode, int maxit, int qlim,
   hipLaunchKernelGGL(k_mismatch_mb, xgrid(e->T, e->n, e->mis_threads),
                      dim3(e->mis_threads), 0, e->stream, e->g, e->d, mode,
                      fd_norm, e->opt.qlim_tol, qlim);
-  // 1024 lanes: the reactive-limit switching walks every bus of an instance
-  hipLaunchKernelGGL(k_verdict, dim3(e->T), dim3(1024), 0, e->stream, e->g, e->d,
+  // 1024 lanes where the reactive-limit switching may walk every bus of an
+  // instance; else one wave for the partial norms (1500 instances of 1354 buses
+  // 22 us with 1024 lanes, 15 with 64)
+  hipLaunchKernelGGL(k_verdict, dim3(e->T), dim3(qlim ? 1024 : 64), 0, e->stream, e->g, e->d,
                      (int)nparts, mode, maxit, e->opt.tol, qlim,
                      e->opt.max_qlim_rounds, e->opt.qlim_tol, fd_norm);
 }

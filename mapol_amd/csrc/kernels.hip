@@ -505,18 +505,20 @@ __global__ void k_verdict(DevTopo g, DevInst d, int nparts, int mode, int maxit,
   if (mode != 2 && sp->done) return;
   double pm = 0.0;
   int pn = 0, pv = 0;
-  for (int q = threadIdx.x; q < nparts; q += blockDim.x) {
+  // every wave reduces all the partials (a few dozen), so none waits for another
+  for (int q = threadIdx.x & 63; q < nparts; q += 64) {
     double v = d.part[(size_t)t * nparts + q];
     pn |= isnan(v);
     pm = fmax(pm, v);
     pv += d.partv[(size_t)t * nparts + q];
   }
-  double nrm = block_max(pm, shd);
-  int anynan = block_or(pn, shi);
+  double nrm = wave_max(pm);
+  int anynan = wave_or(pn);
   // PV buses beyond their reactive limits at this V (counted per bus by the
   // mismatch kernel); after a switch the remaining ones are recounted here
-  int nviol_at_v = enforce_qlim ? block_add(pv, shi) : 0;
+  int nviol_at_v = enforce_qlim ? wave_add(pv) : 0;
   InstState s = *sp;
+  __syncthreads();    // every wave has read the state that the first one replaces
   const bool active = verdict_of(g, d, t, nrm, anynan, nviol_at_v, mode, maxit, tol, enforce_qlim,
                                  max_rounds, qtol, fd_norm, shd, shi, s);
   if (threadIdx.x == 0) {
