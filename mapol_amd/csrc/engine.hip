@@ -427,11 +427,41 @@ static bpf_status bus_rows_upload(bpf_engine *e, const cd *src, cd *ddst, size_t
   return BPF_OK;
 }
 
-// the LDS-resident plan of one precision, uploaded as one buffer
-static bpf_status build_resident_plan(bpf_engine *e, int fp64) {
-  ResidentPlan H;
-  const int sc = fp64 ? 8 : 4;
-  build_resident(e->S, resident_cap(RES_TOP_LDS, sc), resident_cap(RES_SMALL_LDS, sc), H);
+// the LDS-resident plans, built beside the rest of bpf_create (a plan takes 0.8
+// ms of host time at 1354 buses and 8 at 9241; below 64 blocks a thread costs
+// more than the plan).  Without memory for a plan the chunks run.
+struct ResidentJobs {
+  ResidentPlan H[2];
+  std::thread th[2];
+  void start(const Symbolic &S, int fp64) {
+    auto run = [this, &S, fp64] {
+      const int sc = fp64 ? 8 : 4;
+      try {
+        build_resident(S, resident_cap(RES_TOP_LDS, sc), resident_cap(RES_SMALL_LDS, sc),
+                       H[fp64]);
+      } catch (const std::exception &) {
+        H[fp64].ok = false;
+      }
+    };
+    if (S.nb >= 64) {
+      try {
+        th[fp64] = std::thread(run);
+        return;
+      } catch (const std::exception &) {
+      }
+    }
+    run();
+  }
+  void join(int fp64) {
+    if (th[fp64].joinable()) th[fp64].join();
+  }
+  ~ResidentJobs() { join(0); join(1); }
+};
+
+// the plan of one precision, uploaded as one buffer
+static bpf_status upload_resident_plan(bpf_engine *e, ResidentJobs &jobs, int fp64) {
+  jobs.join(fp64);
+  const ResidentPlan &H = jobs.H[fp64];
   if (!H.ok) return BPF_OK;
   ResPlan &R = e->res[fp64];
   const std::vector<int> word(H.word.begin(), H.word.end()), desc(H.desc.begin(), H.desc.end());
@@ -575,6 +605,9 @@ extern "C" bpf_status bpf_create(const bpf_case *c, const bpf_options *o,
       e->yx_row[r + 1] = (int)e->yx_col.size();
     }
   }
+  ResidentJobs jobs;
+  jobs.start(e->S, 1);
+  if (e->opt.precision == BPF_MIXED) jobs.start(e->S, 0);
   // device
   const char *dbg = getenv("BPF_DEBUG_SYNC");
   e->debug_sync = (dbg && dbg[0] == '1') ? 1 : 0;
@@ -646,7 +679,6 @@ extern "C" bpf_status bpf_create(const bpf_case *c, const bpf_options *o,
       hipLaunchKernelGGL(k_branch_pre, dim3(div_up(e->m, 256)), dim3(256), 0,
                          e->stream, g, (cd *)p1, (cd *)p2);
       HIPCHK(hipGetLastError());
-      HIPCHK(hipStreamSynchronize(e->stream));
     }
     g.ys = (const cd *)p1;
     g.ejs = (const cd *)p2;
@@ -837,8 +869,8 @@ extern "C" bpf_status bpf_create(const bpf_case *c, const bpf_options *o,
     SP.sl_nfw_t = S.sl_nfw_t;
     SP.sl_nbw_t = S.sl_nbw_t;
   }
-  if ((s = build_resident_plan(e, 1))) return s;
-  if (e->opt.precision == BPF_MIXED && (s = build_resident_plan(e, 0))) return s;
+  if ((s = upload_resident_plan(e, jobs, 1))) return s;
+  if (e->opt.precision == BPF_MIXED && (s = upload_resident_plan(e, jobs, 0))) return s;
   e->sweep_form = 0;
   e->tail_form = BPF_TAIL_MFMA;
 #undef UP
