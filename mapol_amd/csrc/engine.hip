@@ -683,33 +683,6 @@ extern "C" bpf_status bpf_create(const bpf_case *c, const bpf_options *o,
     g.ys = (const cd *)p1;
     g.ejs = (const cd *)p2;
   }
-  {
-    // the entries at the case's own taps (another tap computes its entry)
-    const size_t cnt = 4 * (size_t)std::max(e->m, 1);
-    void *p1, *p2 = nullptr;
-    std::vector<int> at(4 * (size_t)std::max(e->m, 1));
-    for (const auto &l : {std::make_pair(&S.yf_ptr, &S.yf_item), std::make_pair(&S.yt_ptr, &S.yt_item)})
-      for (int p = 0; p < g.nnzY; p++)
-        for (int q = (*l.first)[p]; q < (*l.first)[p + 1]; q++) at[(*l.second)[q]] = p;
-    const std::vector<uint8_t> on0(e->br_status);
-    UP(g.tap0, nonemptyd(e->tap)); UP(g.on0, nonempty8(on0)); UP(g.ybr, at);
-    void *p3;
-    if ((s = dalloc(e, e->owned, sizeof(cd) * cnt, &p1))) return s;
-    if (e->opt.alg != BPF_NR && (s = dalloc(e, e->owned, sizeof(double2) * cnt, &p2))) return s;
-    if ((s = dalloc(e, e->owned, sizeof(cd) * (size_t)g.nnzY, &p3))) return s;
-    if (e->m) {
-      hipLaunchKernelGGL(k_branch_entries, dim3(div_up(cnt, 256)), dim3(256), 0, e->stream, g,
-                         (int)e->opt.alg, (cd *)p1, (double2 *)p2);
-      HIPCHK(hipGetLastError());
-    }
-    hipLaunchKernelGGL(k_ybus_base, dim3(div_up(g.nnzY, 256)), dim3(256), 0, e->stream, g,
-                       (cd *)p3);
-    HIPCHK(hipGetLastError());
-    HIPCHK(hipStreamSynchronize(e->stream));
-    g.ybase = (const cd *)p3;
-    g.ent = (const cd *)p1;
-    g.ent_fd = (const double2 *)p2;
-  }
   UP(g.Gs, e->Gs); UP(g.Qd, e->Qd); UP(g.Va0, e->Va);
   UP(g.base_type, e->bus_type);
   {
@@ -733,6 +706,34 @@ extern "C" bpf_status bpf_create(const bpf_case *c, const bpf_options *o,
     UP(ca.Qmax, nonemptyd(e->Qmax)); UP(ca.Qmin, nonemptyd(e->Qmin));
     UP(ca.VG, nonemptyd(e->VG)); UP(ca.gen_status, nonempty8(gst));
     ca.ng = e->ng;
+  }
+  {
+    // the entries at the case's own taps (another tap computes its entry)
+    const size_t cnt = 4 * (size_t)std::max(e->m, 1);
+    void *p1, *p2 = nullptr;
+    std::vector<int> at(4 * (size_t)std::max(e->m, 1));
+    for (const auto &l : {std::make_pair(&S.yf_ptr, &S.yf_item), std::make_pair(&S.yt_ptr, &S.yt_item)})
+      for (int p = 0; p < g.nnzY; p++)
+        for (int q = (*l.first)[p]; q < (*l.first)[p + 1]; q++) at[(*l.second)[q]] = p;
+    UP(g.ybr, at);
+    g.tap0 = e->ca.tap;
+    g.on0 = e->ca.br_status;
+    void *p3;
+    if ((s = dalloc(e, e->owned, sizeof(cd) * cnt, &p1))) return s;
+    if (e->opt.alg != BPF_NR && (s = dalloc(e, e->owned, sizeof(double2) * cnt, &p2))) return s;
+    if ((s = dalloc(e, e->owned, sizeof(cd) * (size_t)g.nnzY, &p3))) return s;
+    if (e->m) {
+      hipLaunchKernelGGL(k_branch_entries, dim3(div_up(cnt, 256)), dim3(256), 0, e->stream, g,
+                         (int)e->opt.alg, (cd *)p1, (double2 *)p2);
+      HIPCHK(hipGetLastError());
+    }
+    hipLaunchKernelGGL(k_ybus_base, dim3(div_up(g.nnzY, 256)), dim3(256), 0, e->stream, g,
+                       (cd *)p3);
+    HIPCHK(hipGetLastError());
+    HIPCHK(hipStreamSynchronize(e->stream));
+    g.ybase = (const cd *)p3;
+    g.ent = (const cd *)p1;
+    g.ent_fd = (const double2 *)p2;
   }
   FactorPlan &F = e->fplan;
   F.nchunk = S.nchunk;
