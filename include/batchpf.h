@@ -459,6 +459,14 @@ bpf_status bpf_set_schedule(bpf_engine *e, int32_t newton_per_graph,
  * gives every part a workgroup at any count. */
 bpf_status bpf_set_factor_split(bpf_engine *e, int32_t workgroups);
 
+/* The form that the engine's last factorization (of a Newton step, the
+ * decoupled matrices or the adjoint) took: BPF_FACTOR_LDS from LDS in parts,
+ * BPF_FACTOR_CHUNKS in chunks of products (other than 1024 lanes, the tail on
+ * the vector ALUs, or an elimination tree that does not divide into parts);
+ * -1 before the first one. */
+enum { BPF_FACTOR_CHUNKS = 0, BPF_FACTOR_LDS = 1 };
+int32_t bpf_factor_form(const bpf_engine *e);
+
 /* Forward substitution inside the factorization (no counterpart in the
  * reference, whose solves run both sweeps): while at most `max_active`
  * instances of a batch part are active, the Newton step's factorization

@@ -153,6 +153,7 @@ struct bpf_engine {
   int graph_fallback = 0;      // the last solve abandoned replay (graph_err says why)
   int graph_captures = 0;      // captures since bpf_create
   int fused_forward = 0;       // the last Newton step's first solve skipped the forward sweep
+  int factor_form = -1;        // the last factorization: BPF_FACTOR_CHUNKS / BPF_FACTOR_LDS
   // timing
   int timing = 0;
   std::vector<TimedEvent> events;
@@ -1269,6 +1270,7 @@ static void launch_resident(bpf_engine *e, B4<T> *LU, B4<T> *TL, B4<T> *UPD, int
   const ResPlan &R = e->res[fp64];
   const std::vector<int> &sg = e->res_stage[fp64];
   const int last = (int)sg.size() - 2;
+  e->factor_form = BPF_FACTOR_LDS;
   for (int q = 0; q < last; q++)
     hipLaunchKernelGGL(k_res_parts<T>, dim3((unsigned)e->T * (sg[q + 1] - sg[q])),
                        dim3(RES_SMALL_LANES), 0, e->stream, e->g, (const InstState *)e->d.st, R,
@@ -1284,6 +1286,7 @@ static void factor_fp64(bpf_engine *e, B4<double> *LU, B4<double> *TL) {
     launch_resident<double>(e, LU, TL, UPD, 0, 0);
     return;
   }
+  e->factor_form = BPF_FACTOR_CHUNKS;
   hipLaunchKernelGGL(k_lu_factor<double>, dim3(e->T), dim3(e->lu_threads), 0, e->stream,
                      e->g, e->d.st, 0, e->fplan, LU, TL, 0, e->d.jsing, 0, nullptr, 0, -1);
 }
@@ -1309,6 +1312,7 @@ static void launch_newton_step(bpf_engine *e) {
   // whatever the active count, so the limit is the caller's or none
   if (resident && fused && !e->fused_set) fp.fused_limit = 1 << 20;
   e->fused_forward = fused ? fp.fused_limit : -1;
+  if (!resident) e->factor_form = BPF_FACTOR_CHUNKS;
   tbegin(e, "jacobian");
   hipLaunchKernelGGL(k_jacobian<T>, xgrid(e->T, ((size_t)e->g.nJb + 1) / 2, 256),
                      dim3(256), 0, e->stream, e->g, e->d, LU, c0 > 0 ? 1 : 0,
@@ -1454,6 +1458,8 @@ static void launch_loss(bpf_engine *e, const int *gate, int *count) {
 static bpf_status run_newton(bpf_engine *e, bool *graph_failed, bool *loss_done) {
   bpf_status s = ensure_lu(e, e->opt.precision == BPF_FP64 ? 1 : 0);
   if (s) return s;
+  // (a graph replayed below was captured with this form)
+  e->factor_form = resident_runs(e, e->lu_fp64) ? BPF_FACTOR_LDS : BPF_FACTOR_CHUNKS;
   // per-kernel timing uses events around direct launches: elapsed times
   // between event nodes of a replayed graph are not reliable on this runtime
   bool use_graph = e->opt.use_graph != 0 && !e->graph_broken && !e->timing;
@@ -2075,6 +2081,10 @@ extern "C" bpf_status bpf_get_info(const bpf_engine *e, bpf_info *info) {
   int fp64 = e->opt.precision == BPF_FP64;
   info->lds_solve = ((fp64 ? 8 : 4) * 2 * (size_t)S.nb) <= (size_t)SOLVE_LDS_BYTES;
   return BPF_OK;
+}
+
+extern "C" int32_t bpf_factor_form(const bpf_engine *e) {
+  return e ? e->factor_form : -1;
 }
 
 extern "C" bpf_status bpf_set_timing(bpf_engine *e, int32_t enable) {

@@ -17,6 +17,7 @@ BPF_NR, BPF_FDXB, BPF_FDBX = 0, 1, 2
 BPF_FP64, BPF_MIXED = 0, 1
 CONVERGED, MAX_ITER, SINGULAR, NONFINITE = 0, 1, 2, 3
 CTL_AVR, CTL_OLTC, CTL_SHC = 1, 2, 3
+FACTOR_CHUNKS, FACTOR_LDS = 0, 1
 
 _pi = C.POINTER(C.c_int32)
 _pd = C.POINTER(C.c_double)
@@ -33,6 +34,7 @@ EXPORTS = [
     "bpf_adjoint",
     "bpf_set_timing", "bpf_get_kernel_time", "bpf_set_launch",
     "bpf_set_schedule", "bpf_set_factor_split", "bpf_set_fused_forward",
+    "bpf_factor_form",
     "bpf_analyse", "bpf_analyse_sweeps", "bpf_analyse_fill", "bpf_analyse_tail",
     "bpf_analyse_slots", "bpf_analyse_slots_transposed",
     "bpf_load_matpower",
@@ -135,6 +137,7 @@ def load_library(path: str = LIB_PATH):
     L.bpf_set_schedule.argtypes = [V, C.c_int32, C.c_int32, C.c_int32, C.c_int32]
     L.bpf_set_factor_split.argtypes = [V, C.c_int32]
     L.bpf_set_fused_forward.argtypes = [V, C.c_int32]
+    L.bpf_factor_form.argtypes = [V]
     L.bpf_analyse.argtypes = [C.POINTER(BpfCase), C.POINTER(BpfInfo)] + [_pi] * 21
     L.bpf_analyse_sweeps.argtypes = [C.POINTER(BpfCase), C.POINTER(BpfInfo)] + [_pi] * 3
     L.bpf_analyse_fill.argtypes = [C.POINTER(BpfCase), C.POINTER(BpfInfo)] + [_pi] * 2
@@ -627,6 +630,11 @@ class Engine:
         2 / 4 / 8 always"""
         self._check(self.L.bpf_set_factor_split(self.h, int(workgroups)),
                     "bpf_set_factor_split")
+
+    def factor_form(self):
+        """the last factorization's form (``bpf_factor_form``): FACTOR_LDS,
+        FACTOR_CHUNKS, or -1 before the first one"""
+        return int(self.L.bpf_factor_form(self.h))
 
     def set_launch(self, lu=0, solve=0, mismatch=0):
         self._check(self.L.bpf_set_launch(self.h, lu, solve, mismatch),
