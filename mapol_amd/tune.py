@@ -7,19 +7,24 @@ What it picks, per case topology, instance count and precision:
   analysis): minimum degree or its least-height equivalent, pivots of the
   dense tail
   (``tail_limit``), block products per factorization chunk
-  (``chunk_products``) and lane slots per slot-form sweep chunk
+  (``chunk_products``; left at its default where the factorization runs from
+  LDS, which has no such chunks) and lane slots per slot-form sweep chunk
   (``slot_chunk``);
 * launch shapes (``bpf_set_launch``): workgroup sizes of the factorization,
   the sweeps and the mismatch, timed per kernel family with HIP events;
 * the run-time schedule (``bpf_set_schedule``): Newton iterations per
-  captured graph, the dense-tail inverse on matrix cores or vector ALUs and
-  the number of concurrent parts the batch runs as.
+  captured graph, the dense-tail inverse on matrix cores or vector ALUs (the
+  latter, like other than 1024 factorization lanes, takes the whole
+  factorization in chunks of products instead of from LDS) and the number of
+  concurrent parts the batch runs as.
 
 Tiles and schedule are judged by the wall time of whole batched solves (they
 move time between kernels), the launch shapes by their own kernel's time.
 The search is coordinate descent in the order above, starting from the
-engine's defaults.  Results persist in a JSON cache keyed by
-:func:`signature`; a cached entry is applied without measuring.
+engine's defaults (the first candidate of each list).  Results persist in a
+JSON cache keyed by :func:`signature`; a cached entry is applied without
+measuring.  The key names the kernels' generation (``KERNELS``): what was
+measured on other kernels is not applied to these.
 """
 from __future__ import annotations
 
@@ -28,11 +33,17 @@ import os
 import time
 import zlib
 
+from .engine import FACTOR_LDS
+
+# generation of the kernels an entry was measured on: raised when a kernel or a
+# default changes which choices are the fastest (2: factorization from LDS,
+# 1024-slot sweep chunks)
+KERNELS = 2
 TILE_CANDIDATES = {
     "ordering": (0, 1),            # minimum degree; its least-height reorder
     "tail_limit": (64, 56, 48, 40),
     "chunk_products": (4096, 3072, 2048),
-    "slot_chunk": (2048, 1024, 512),
+    "slot_chunk": (1024, 2048, 512),
 }
 SCHEDULE_CANDIDATES = {
     "newton_per_graph": (4, 2, 8),
@@ -40,7 +51,7 @@ SCHEDULE_CANDIDATES = {
     "parts": (1, 2, 4),            # concurrent parts of the batch
     # the forward substitution in the factorization while at most this
     # many instances of a part are active (-1 never, 1 << 20 always)
-    "fused_forward": (32, -1, 8, 64, 1 << 20),
+    "fused_forward": (1 << 20, -1, 8, 32, 64),
 }
 CANDIDATES = (256, 512, 1024)      # workgroup sizes
 FAMILIES = {"lu": "lu_factor", "solve": "lu_solve", "mismatch": "mismatch"}
@@ -50,13 +61,13 @@ DEFAULT_CACHE = os.path.join(os.path.dirname(os.path.abspath(__file__)),
 
 def signature(case, T, precision, refine, qlim) -> str:
     """cache key: sizes, a CRC of the topology and bus types, the instance
-    count and the numerical settings"""
+    count, the numerical settings and the kernels' generation"""
     import numpy as np
     h = zlib.crc32(np.ascontiguousarray(case.br_from, np.int32).tobytes())
     h = zlib.crc32(np.ascontiguousarray(case.br_to, np.int32).tobytes(), h)
     h = zlib.crc32(np.ascontiguousarray(case.bus_type, np.int32).tobytes(), h)
     return (f"n{case.nbus}-m{case.nbranch}-{h:08x}-T{int(T)}-p{int(precision)}-"
-            f"r{int(refine)}-q{int(bool(qlim))}")
+            f"r{int(refine)}-q{int(bool(qlim))}-k{KERNELS}")
 
 
 def load_cache(path):
@@ -86,6 +97,12 @@ def _solve_ms(engine, reps):
         ts.append(time.perf_counter() - t0)
     ts.sort()
     return 1e3 * ts[len(ts) // 2]
+
+
+def _in_lds(engine):
+    """whether the engine's last factorization ran from LDS"""
+    form = getattr(engine, "factor_form", None)
+    return form is not None and form() == FACTOR_LDS
 
 
 def _avg_us(engine, kernel):
@@ -153,9 +170,11 @@ def tune(make_engine, key, cache_path=DEFAULT_CACHE, reps=3, verbose=False,
 
     # 1. tiles: one engine per candidate, whole solves
     tiles = {k: v[0] for k, v in tile_candidates.items()}
-    best_ms = None
+    best_ms, in_lds = None, False
     for name, cands in tile_candidates.items():
         res = {}
+        if name == "chunk_products" and in_lds:
+            continue
         for c in cands:
             t = dict(tiles, **{name: c})
             try:
@@ -166,6 +185,7 @@ def tune(make_engine, key, cache_path=DEFAULT_CACHE, reps=3, verbose=False,
                 continue
             try:
                 res[c] = _solve_ms(e, reps)
+                in_lds = _in_lds(e)
             finally:
                 e.close()
             trials.append(dict(stage="tiles", tiles=t, ms=round(res[c], 3)))
