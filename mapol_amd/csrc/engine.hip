@@ -1582,21 +1582,34 @@ static bpf_status run_newton(bpf_engine *e, bool *graph_failed, bool *loss_done)
   return BPF_OK;
 }
 
+// The whole decoupled loop in one launch (k_fd_one), a workgroup and compute
+// unit per instance: not for so many buses that their mismatch needs more than
+// one compute unit, nor for many small instances, which the launches keep
+// several to a compute unit.  A solve, time by launches over time in one, by
+// instances (256 compute units):
+//    buses      1     32    100    256    512    768   1024   1280   1500
+//       14   2.63                2.95   1.98   1.64   1.40   1.30   1.19
+//       64                              1.47   1.32   1.16   1.12   1.04
+//      118   1.79         1.95   1.78   1.25   1.12   0.91   0.90   0.82
+//      350                              1.10   1.02   0.93   0.92   0.89
+//      700                                     1.12   1.01   1.00   0.98
+//     1354   1.15         1.21   1.25   1.03   1.11   0.99   1.00   0.98
+//     2000   1.05         1.13   1.13   1.21   1.26   1.22   1.26   1.17
+//     2450   1.01   1.00   1.07   1.04   1.00
+//     2869   0.95   0.95   1.02   1.00   1.02
+//     3000   0.95   0.95   1.03   1.02   0.95
+//     3300   0.92   0.92   0.98   1.00   0.93
+//     4096   0.86          0.94   0.98
+// (the rows' spread is their slowest instance: launches repeat for it alone)
+static bool fd_one(const bpf_engine *e) {
+  if (e->n < 700) return e->T <= (e->n <= 64 ? 6 : 3) * e->num_cu;
+  return e->n <= 2500 || (e->n <= 3000 && e->T >= e->num_cu / 4);
+}
+
 // fast decoupled (mkl_fdpf, fdpf.h:450-596): B' and B'' of every instance
 // assembled and factored once in FP64, then P and Q half-steps; each half-step
 // is a masked solve with the same factors, an update and the |V|-normalised
 // mismatch with the reference's convergence checks
-// The whole decoupled loop in one launch (k_fd_one), a workgroup and compute
-// unit per instance: not for so many buses that their mismatch needs more than
-// one compute unit, nor for many small instances, which the launches keep
-// several to a compute unit.  A solve, launches / one: 14 buses x 1 432 / 158
-// us, 118 x 1 838 / 436, 118 x 2000 3979 / 4265, 1354 x 1 817 / 678, x 200
-// 1508 / 1173, x 1000 4683 / 4087, 2869 x 100 1613 / 1560, 9241 x 1 2025 /
-// 2881, x 200 7023 / 8060.
-static bool fd_one(const bpf_engine *e) {
-  return e->n <= 4096 && (e->n >= 1024 || e->T <= 4 * e->num_cu);
-}
-
 static bpf_status run_fd(bpf_engine *e) {
   B4<double> *LU, *TLd;
   double *xg;
