@@ -1198,16 +1198,27 @@ static void launch_mismatch(bpf_engine *e, int mode) {
 }
 
 // Lanes of a solve's workgroup, unless the caller chose them.  1024 lanes fill a
-// compute unit with one instance; with more instances than compute units the
+// compute unit with one instance; with many more instances than compute units the
 // slot form takes 256 and four slots a lane where three such workgroups fit the
 // LDS, and the chunks' barriers and round trips of several instances overlap.
 // A pass, 1024 / 256 lanes: 1354 buses x 200 26 / 32 us, x 400 47 / 35, x 1500
 // 153 / 91, in FP64 164 / 141; 2869 x 600 110 / 87; 118 x 2000 64 / 41; 9241 x
 // 600, one workgroup either way, 321 / 454.
+// A solve ends with a few instances, for which the wide form is the faster, and
+// more so the longer its sweeps; so the count that pays grows with the buses
+// (n / 6), and with reactive limits, where most iterations have few instances,
+// further (3 n / 4).  Whole mixed-precision solves, 1024 / 256 lanes in us:
+//   118 buses x 257       661 / 631      with limits 671 / 647
+//   1354 x 257, 400       1135 / 1135, 1375 / 1328     5100 / 5428, 6765 / 7065
+//   1354 x 1000, 1500     2730 / 2580, 4000 / 3651     9590 / 9590, 13000 / 12450
+//   2869 x 300, 600       2025 / 2141, 3550 / 3492     2840 / 3020, 4328 / 4400
+//   4096 x 300            2320 / 2331                  7797 / 8787
 static int solve_lanes(const bpf_engine *e, size_t scalar) {
   const size_t xs = scalar * 2 * (size_t)e->S.nb, lds = xs + SOLVE_LDS_FIXED;
+  const long long T = (long long)e->T * std::max(1, e->parts_running);
+  const long long pays = e->opt.enforce_qlim ? 3LL * e->n / 4 : e->n / 6;
   return !e->solve_set && e->solve_threads == 1024 &&
-                 e->T * std::max(1, e->parts_running) > e->num_cu &&
+                 T > std::max<long long>(e->num_cu, pays) &&
                  3 * lds <= (size_t)160 * 1024 && e->S.prm.slot_chunk <= 1024 &&
                  sweep_mode(e->S, scalar, 1, e->sweep_form, 1024) == 2
              ? 256
