@@ -119,7 +119,8 @@ struct bpf_engine {
   struct Fp64Factors { void *LU = nullptr, *TL = nullptr, *xglob = nullptr, *UPD = nullptr; } f64;
   // LDS-resident factorization, per precision (0 FP32: mixed Newton steps, 1
   // FP64): the plan, its first part of each stage (empty: the tree does not
-  // fit it), and the Newton factors' updates between parts [T][2 * nupd]
+  // fit it), and the Newton factors' updates between parts [T][2 * nupd] (null
+  // where there is no memory for them)
   ResPlan res[2]{};
   std::vector<int> res_stage[2];
   void *d_UPD = nullptr;
@@ -201,11 +202,39 @@ static void drop_graphs(bpf_engine *e) {
     }                                                                       \
   } while (0)
 
+// the updates between the parts of the LDS-resident factorization, given back:
+// without them it runs in chunks.  (hipFree waits for the kernels using them.)
+static bool release_updates(bpf_engine *e) {
+  bool any = false;
+  for (void **q : {&e->d_UPD, &e->f64.UPD}) {
+    if (!*q) continue;
+    for (auto it = e->inst_owned.begin(); it != e->inst_owned.end(); ++it)
+      if (it->p == *q) { hipFree(it->p); e->inst_owned.erase(it); break; }
+    *q = nullptr;
+    any = true;
+  }
+  if (any) drop_graphs(e);
+  return any;
+}
+
+// device memory; what a call cannot do without takes the updates' place
+static hipError_t device_alloc(bpf_engine *e, void **p, size_t bytes) {
+  hipError_t r = hipMalloc(p, bytes);
+  if (r == hipErrorOutOfMemory) {
+    (void)hipGetLastError();
+    if (release_updates(e)) {
+      r = hipMalloc(p, bytes);
+      if (r != hipSuccess) (void)hipGetLastError();
+    }
+  }
+  return r;
+}
+
 static bpf_status dalloc(bpf_engine *e, std::vector<DBuf> &pool, size_t bytes,
                          void **out) {
   void *p = nullptr;
   if (bytes == 0) bytes = 16;
-  hipError_t r = hipMalloc(&p, bytes);
+  hipError_t r = device_alloc(e, &p, bytes);
   if (r != hipSuccess) {
     e->err = "hipMalloc(" + std::to_string(bytes) + "): " + hipGetErrorString(r);
     return r == hipErrorOutOfMemory ? BPF_ERR_OOM : BPF_ERR_HIP;
@@ -307,7 +336,7 @@ static bpf_status bus_stage(bpf_engine *e, size_t bytes) {
   if (e->d_bus_stage) HIPCHK(hipFree(e->d_bus_stage));
   e->d_bus_stage = nullptr;
   e->bus_stage_bytes = 0;
-  HIPCHK(hipMalloc(&e->d_bus_stage, bytes));
+  HIPCHK(device_alloc(e, &e->d_bus_stage, bytes));
   e->bus_stage_bytes = bytes;
   return BPF_OK;
 }
@@ -1070,6 +1099,24 @@ extern "C" bpf_status bpf_set_instances(bpf_engine *e, int32_t T,
   return BPF_OK;
 }
 
+// the updates of T instances, or null where there is no memory for them
+static bpf_status alloc_updates(bpf_engine *e, int fp64, void **out) {
+  *out = nullptr;
+  if (e->res_stage[fp64].empty()) return BPF_OK;
+  const size_t el = fp64 ? sizeof(B4<double>) : sizeof(B4<float>);
+  const size_t bytes = std::max<size_t>(16, el * (size_t)e->T * 2 * e->res[fp64].nupd);
+  void *p = nullptr;
+  const hipError_t r = hipMalloc(&p, bytes);
+  if (r == hipErrorOutOfMemory) {
+    (void)hipGetLastError();
+    return BPF_OK;
+  }
+  HIPCHK(r);
+  e->inst_owned.push_back({p, bytes});
+  *out = p;
+  return BPF_OK;
+}
+
 // (re)allocate the factor storage for the requested precision
 static bpf_status ensure_lu(bpf_engine *e, int fp64) {
   if (e->lu_fp64 == fp64 && e->d_LU) return BPF_OK;
@@ -1088,8 +1135,6 @@ static bpf_status ensure_lu(bpf_engine *e, int fp64) {
   size_t el = fp64 ? sizeof(B4<double>) : sizeof(B4<float>);
   s = dalloc(e, e->inst_owned, el * (size_t)e->T * e->g.nnzLU, &e->d_LU);
   if (s) return s;
-  s = dalloc(e, e->inst_owned, el * (size_t)e->T * 2 * e->res[fp64].nupd, &e->d_UPD);
-  if (s) return s;
   s = dalloc(e, e->inst_owned, el * (size_t)e->T * e->S.tail_n * e->S.tail_n,
              &e->d_TL);
   if (s) return s;
@@ -1098,6 +1143,7 @@ static bpf_status ensure_lu(bpf_engine *e, int fp64) {
     s = dalloc(e, e->inst_owned, xs * e->T, &e->d_xglob);
     if (s) return s;
   }
+  if ((s = alloc_updates(e, fp64, &e->d_UPD))) return s;
   e->lu_fp64 = fp64;
   drop_graphs(e);
   return BPF_OK;
@@ -1121,10 +1167,10 @@ static bpf_status fp64_factors(bpf_engine *e, B4<double> **LU, B4<double> **TL,
     bpf_status s = dalloc(e, e->inst_owned, el * (size_t)e->T * e->g.nnzLU, &f.LU);
     if (!s) s = dalloc(e, e->inst_owned,
                        el * (size_t)e->T * e->S.tail_n * e->S.tail_n, &f.TL);
-    if (!s) s = dalloc(e, e->inst_owned, el * (size_t)e->T * 2 * e->res[1].nupd, &f.UPD);
     const size_t xs = sizeof(double) * 2 * (size_t)e->S.nb;
     if (!s && xs > (size_t)SOLVE_LDS_BYTES)
       s = dalloc(e, e->inst_owned, xs * e->T, &f.xglob);
+    if (!s) s = alloc_updates(e, 1, &f.UPD);
     if (s) { f = bpf_engine::Fp64Factors(); return s; }
   }
   *LU = (B4<double> *)f.LU;
@@ -1265,11 +1311,18 @@ static void launch_solve(bpf_engine *e, int T_, const void *LU, int rhs_mode,
   }
 }
 
+// the updates of a precision's factors: FP64 factors of a mixed engine are a
+// second set
+static void *updates_of(const bpf_engine *e, int fp64) {
+  return fp64 && e->opt.precision != BPF_FP64 ? e->f64.UPD : e->d_UPD;
+}
+
 // the LDS-resident form of the factorization (1024 lanes, tail on the matrix
-// cores); the other launch shapes and the vector-ALU tail keep the chunks
+// cores); the other launch shapes and the vector-ALU tail keep the chunks, and
+// so does a batch without memory for the updates
 static bool resident_runs(const bpf_engine *e, int fp64) {
   return !e->res_stage[fp64].empty() && e->lu_threads == RES_TOP_LANES &&
-         e->fplan.tail_mfma;
+         e->fplan.tail_mfma && updates_of(e, fp64);
 }
 
 // every part of a stage and instance its own workgroup, one launch a stage;
@@ -1293,8 +1346,7 @@ static void launch_resident(bpf_engine *e, B4<T> *LU, B4<T> *TL, B4<T> *UPD, int
 // FP64 factorization outside the Newton step (level 0 included)
 static void factor_fp64(bpf_engine *e, B4<double> *LU, B4<double> *TL) {
   if (resident_runs(e, 1)) {
-    B4<double> *UPD = (B4<double> *)(e->opt.precision == BPF_FP64 ? e->d_UPD : e->f64.UPD);
-    launch_resident<double>(e, LU, TL, UPD, 0, 0);
+    launch_resident<double>(e, LU, TL, (B4<double> *)updates_of(e, 1), 0, 0);
     return;
   }
   e->factor_form = BPF_FACTOR_CHUNKS;
@@ -1421,7 +1473,7 @@ static PartView part_view(bpf_engine *e, int h, int K) {
   const size_t tn = e->S.tail_n;
   v.LU = (char *)e->d_LU + o * el * e->g.nnzLU;
   v.TL = (char *)e->d_TL + o * el * tn * tn;
-  v.UPD = (char *)e->d_UPD + o * el * 2 * e->res[e->lu_fp64 == 1].nupd;
+  v.UPD = e->d_UPD ? (char *)e->d_UPD + o * el * 2 * e->res[e->lu_fp64 == 1].nupd : nullptr;
   v.xg = e->d_xglob ? (char *)e->d_xglob + o * (e->lu_fp64 ? 8 : 4) * nb2 : nullptr;
   v.s = h == 0 ? e->stream : e->sub[h];
   v.hc = e->h_count + h;
