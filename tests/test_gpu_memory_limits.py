@@ -1,14 +1,18 @@
 """Batches at the limit of the device's memory: what does not need the updates of
-the factorization from LDS fits where it fitted without them.  A filler tensor
-leaves room for everything but them (margins of 1 GB and more for the runtime);
-the solve then runs in chunks, or gives them back when a later call needs their
-place, with the same results up to rounding (quadratic convergence to 1e-8:
-1e-9)."""
+the factorization from LDS fits where it fitted without them.  An allocation
+beside the engine leaves room for everything but them (margins of 1 GB and more
+for the runtime); the solve then runs in chunks, or gives them back when a later
+call needs their place, with the same results up to rounding (quadratic
+convergence to 1e-8: 1e-9)."""
+import contextlib
+import ctypes as C
+
 import numpy as np
 import pytest
 
 from mapol_amd import synth
-from mapol_amd.engine import BPF_FP64, BPF_MIXED, FACTOR_CHUNKS, FACTOR_LDS, Engine
+from mapol_amd.engine import (BPF_FP64, BPF_MIXED, FACTOR_CHUNKS, FACTOR_LDS, Engine,
+                              load_library)
 
 pytestmark = pytest.mark.gpu
 
@@ -41,19 +45,31 @@ def _mesh(k):
                  np.r_[q[:, 1:].ravel(), q[1:].ravel()], 4e-4)
 
 
-def _fill(leave):
-    """all of the device's free memory but `leave` bytes"""
-    import torch
-    torch.cuda.synchronize()
-    free = torch.cuda.mem_get_info()[0]
-    assert free > leave
-    return torch.empty(free - leave, dtype=torch.uint8, device="cuda")
+def _hip():
+    """the HIP runtime that the engine's library runs on"""
+    L = load_library()
+    L.hipMalloc.argtypes = [C.POINTER(C.c_void_p), C.c_size_t]
+    L.hipFree.argtypes = [C.c_void_p]
+    L.hipMemGetInfo.argtypes = [C.POINTER(C.c_size_t)] * 2
+    return L
 
 
 def _free():
-    import torch
-    torch.cuda.synchronize()
-    return torch.cuda.mem_get_info()[0]
+    L, free, total = _hip(), C.c_size_t(), C.c_size_t()
+    assert L.hipDeviceSynchronize() == 0
+    assert L.hipMemGetInfo(C.byref(free), C.byref(total)) == 0
+    return free.value
+
+
+@contextlib.contextmanager
+def _room_for(leave):
+    """all of the device's free memory but `leave` bytes taken"""
+    p = C.c_void_p()
+    assert _hip().hipMalloc(C.byref(p), _free() - leave) == 0
+    try:
+        yield
+    finally:
+        assert _hip().hipFree(p) == 0
 
 
 def _solved(case, T, precision):
@@ -65,9 +81,7 @@ def _solved(case, T, precision):
 
 @pytest.mark.parametrize("precision,T", [(BPF_FP64, 6000), (BPF_MIXED, 10000)])
 def test_no_room_for_the_updates(precision, T):
-    import torch
     case = _mesh(40)
-    torch.cuda.empty_cache()
     free = _free()
     e = _solved(case, T, precision)
     used = free - _free()
@@ -79,15 +93,11 @@ def test_no_room_for_the_updates(precision, T):
     # the updates are more than half of the factors on a mesh: room for all the
     # rest and a quarter of the factors' size
     print(f"[memory] precision {precision}: used {used >> 20} MiB, factors {lu >> 20} MiB", flush=True)
-    hold = _fill(used - lu // 4)
-    try:
+    with _room_for(used - lu // 4):
         e = _solved(case, T, precision)
         assert e.factor_form() == FACTOR_CHUNKS
         got = e.results()
         e.close()
-    finally:
-        del hold
-        torch.cuda.empty_cache()
     for k in ("iterations", "verdict"):
         np.testing.assert_array_equal(got[k], ref[k])
     assert (ref["verdict"] == 0).all()
@@ -95,7 +105,6 @@ def test_no_room_for_the_updates(precision, T):
 
 
 def test_updates_given_back_for_the_adjoint():
-    import torch
     case, T = _mesh(40), 10000
     e = _solved(case, T, BPF_MIXED)
     assert e.factor_form() == FACTOR_LDS
@@ -104,15 +113,11 @@ def test_updates_given_back_for_the_adjoint():
     n, m, nb, lu = case.nbus, case.nbranch, i["nblocks"], i["nnz_lu_blocks"] + i["nblocks"]
     # the adjoint's FP64 factors, tail inverses and arrays
     need = T * (32 * (lu + i["tail_n"] ** 2) + 8 * (4 * nb + 2 * n + m + 8))
-    hold = _fill(need - T * 16 * lu // 4)
-    try:
+    with _room_for(need - T * 16 * lu // 4):
         a = e.adjoint()
         e.solve()
         assert e.factor_form() == FACTOR_CHUNKS
         got = e.results()
-    finally:
-        del hold
-        torch.cuda.empty_cache()
     b = e.adjoint()
     e.close()
     np.testing.assert_array_equal(got["iterations"], ref["iterations"])
