@@ -341,6 +341,19 @@ static bpf_status bus_stage(bpf_engine *e, size_t bytes) {
   return BPF_OK;
 }
 
+// a staging buffer larger than what the voltages of a batch pass through, or
+// than 64 MB, is not kept after the call that needed it
+struct StageTrim {
+  bpf_engine *e;
+  ~StageTrim() {
+    const size_t rows = e->opt.bus_numbering ? sizeof(cd) * (size_t)e->T * e->n : 0;
+    if (e->bus_stage_bytes <= std::max<size_t>(rows, 64u << 20)) return;
+    hipFree(e->d_bus_stage);
+    e->d_bus_stage = nullptr;
+    e->bus_stage_bytes = 0;
+  }
+};
+
 // device memory to the caller's, after the work queued on the engine's stream:
 // through pinned buffers, the copy of one chunk running while the host stores
 // the one before (into pageable memory the runtime does both in turn: 18 GB/s
@@ -1874,7 +1887,9 @@ extern "C" bpf_status bpf_get_branch_loading(bpf_engine *e, const double *rate,
       return BPF_ERR_INVALID_ARG;
     }
   // ratings, counts, largest loadings and rows in the staging buffer, which
-  // the engine keeps (four allocations and their release took 200 us)
+  // the engine keeps (four allocations and their release took 200 us) unless
+  // it is large
+  StageTrim trim{e};
   const size_t o_max = sizeof(double) * std::max(m, 1), o_over = o_max + sizeof(double) * T,
                o_load = (o_over + sizeof(int) * T + 255) / 256 * 256;
   bpf_status s = bus_stage(e, o_load + (loading ? sizeof(double) * (size_t)T * std::max(m, 1) : 0));
