@@ -63,6 +63,11 @@ static int sweep_mode(const Symbolic &S, size_t scalar, int use_lds, int form,
 static dim3 xgrid(int T, size_t count, unsigned threads) {
   return dim3(8u * div_up((size_t)T, 8) * div_up(count, threads));
 }
+// whether that grid's threads can be launched: beyond 2^32 the runtime cuts the
+// grid short without an error
+static bool xgrid_fits(int T, size_t count, unsigned threads) {
+  return 8ull * div_up((size_t)T, 8) * div_up(count, threads) * threads < 1ull << 32;
+}
 
 // results leave through pinned memory: OUT_PARTS copying threads with two
 // buffers of OUT_CHUNK bytes each
@@ -1519,7 +1524,7 @@ struct PartScope {
 // branch flows and losses; gate and count: loss_waits
 static void launch_loss(bpf_engine *e, const int *gate, int *count) {
   const size_t parts = div_up(e->m, 256);
-  if (e->m <= LOSS_ONE || parts > 2 * (size_t)e->S.nb) {
+  if (e->m <= LOSS_ONE || parts > 2 * (size_t)e->S.nb || !xgrid_fits(e->T, e->m, 256)) {
     hipLaunchKernelGGL(k_loss, dim3(e->T), dim3(1024), 0, e->stream, e->g, e->d,
                        e->d_Sf, e->d_St, e->d_loss, gate, count);
   } else {
@@ -1733,9 +1738,11 @@ static bpf_status run_fd(bpf_engine *e) {
 }
 
 static void launch_ybus_changed(bpf_engine *e) {
-  if (e->m)
-    hipLaunchKernelGGL(k_ybus_changed, xgrid(e->T, 4 * (size_t)e->m, 256), dim3(256), 0,
-                       e->stream, e->g, e->d);
+  if (!e->m) return;
+  size_t count = 4 * (size_t)e->m;
+  while (!xgrid_fits(e->T, count, 256)) count /= 2;
+  hipLaunchKernelGGL(k_ybus_changed, xgrid(e->T, count, 256), dim3(256), 0, e->stream, e->g,
+                     e->d, (int)div_up(count, 256));
 }
 
 static bpf_status solve_once(bpf_engine *e, bool *graph_failed) {

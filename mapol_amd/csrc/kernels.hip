@@ -166,16 +166,20 @@ __global__ void k_ybus(DevTopo g, DevInst d) {
   if (t < d.T && p < g.nnzY) ybus_copy(g, d, t, p);
 }
 
-// (a thread per branch and position)
-__global__ void k_ybus_changed(DevTopo g, DevInst d) {
-  const XSlot sl = xcd_slot(parts_of(4 * g.m));
-  const int t = sl.t, q = sl.part * blockDim.x + threadIdx.x, b = q >> 2;
-  if (t >= d.T || b >= g.m) return;
-  const size_t o = (size_t)t * g.m + b;
-  if ((d.br_on[o] != 0) == (g.on0[b] != 0) && d.tap[o] == g.tap0[b]) return;
-  const int p = g.ybr[q];
-  const cd y = ybus_sum(g, p, [&](int it) { return branch_entry(g, d, t, it >> 2, it & 3); });
-  d.Y[(size_t)t * g.nnzY + p] = ybus_shunt(g, d, t, p, y);
+// (a thread per branch and position; `parts` workgroups per instance walk them,
+// all at once but where that would exceed the threads of a launch)
+__global__ void k_ybus_changed(DevTopo g, DevInst d, int parts) {
+  const XSlot sl = xcd_slot(parts);
+  const int t = sl.t;
+  if (t >= d.T) return;
+  for (int q = sl.part * blockDim.x + threadIdx.x; q < 4 * g.m; q += parts * blockDim.x) {
+    const int b = q >> 2;
+    const size_t o = (size_t)t * g.m + b;
+    if ((d.br_on[o] != 0) == (g.on0[b] != 0) && d.tap[o] == g.tap0[b]) continue;
+    const int p = g.ybr[q];
+    const cd y = ybus_sum(g, p, [&](int it) { return branch_entry(g, d, t, it >> 2, it & 3); });
+    d.Y[(size_t)t * g.nnzY + p] = ybus_shunt(g, d, t, p, y);
+  }
 }
 
 // ---------------------------------------------------------------------------
