@@ -138,6 +138,7 @@ struct bpf_engine {
   int *h_count = nullptr;       // pinned
   char *h_out = nullptr;        // pinned, results on their way out (to_host)
   hipEvent_t h_ev[2 * OUT_PARTS] = {};
+  std::mutex out_mu;            // one call at a time has these and the staging buffer
   // launch shapes
   int lu_threads = 1024, solve_threads = 1024, mis_threads = 256;
   int max_lds = 65536;
@@ -1827,6 +1828,7 @@ extern "C" bpf_status bpf_get_results(bpf_engine *e, double *V, int32_t *its,
                                       int32_t *bus_type) {
   if (!e) return BPF_ERR_INVALID_ARG;
   if (!e->solved) { e->err = "no solution yet"; return BPF_ERR_STATE; }
+  std::lock_guard<std::mutex> lock(e->out_mu);
   const size_t T = e->T, n = e->n, cnt = T * n;
   bpf_status s;
   auto states = [&](const InstState *st) {
@@ -1875,6 +1877,7 @@ extern "C" bpf_status bpf_get_results(bpf_engine *e, double *V, int32_t *its,
 extern "C" bpf_status bpf_get_branch_flows(bpf_engine *e, double *Sf, double *St) {
   if (!e) return BPF_ERR_INVALID_ARG;
   if (!e->solved) { e->err = "no solution yet"; return BPF_ERR_STATE; }
+  std::lock_guard<std::mutex> lock(e->out_mu);
   const size_t cnt = (size_t)e->T * e->m;
   bpf_status s;
   if (Sf && (s = to_host(e, e->d_Sf, (cd *)Sf, cnt))) return s;
@@ -1896,6 +1899,7 @@ extern "C" bpf_status bpf_get_branch_loading(bpf_engine *e, const double *rate,
   // ratings, counts, largest loadings and rows in the staging buffer, which
   // the engine keeps (four allocations and their release took 200 us) unless
   // it is large
+  std::lock_guard<std::mutex> lock(e->out_mu);
   StageTrim trim{e};
   const size_t o_max = sizeof(double) * std::max(m, 1), o_over = o_max + sizeof(double) * T,
                o_load = (o_over + sizeof(int) * T + 255) / 256 * 256;
