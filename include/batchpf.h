@@ -417,7 +417,9 @@ bpf_status bpf_adjoint(bpf_engine *e, const double *rate, double w,
 /* Kernel timing on the engine's stream with hipEvents recorded around
  * direct launches (enable before bpf_solve).  While timing is on, the
  * Newton loop launches its kernels directly instead of replaying the
- * iteration graph, so the events bracket single kernels.  Names: ybus, init,
+ * iteration graph, so the events bracket single kernels; the decoupled
+ * method launches its half-steps one by one, also where an untimed solve runs
+ * them all in one kernel (the faster form, not timed here).  Names: ybus, init,
  * mismatch, jacobian, lu_factor, lu_solve, residual, update, loss, bmat,
  * fd_solve, adjoint. */
 bpf_status bpf_set_timing(bpf_engine *e, int32_t enable);
